@@ -24,7 +24,8 @@ LIB_NAME = "libmxfa_mi355x.so"
 LIB_PATH = LIB_DIR / LIB_NAME
 SOURCES = ("split_decode.hip", "split_hd64.hip", "split_hd64_ws.hip", "split_hd64_ws4.hip",
            "split_hd128.hip", "split_hd128_ws.hip", "split_hd128_ws4.hip", "split_hd256.hip",
-           "split_hd256_ws.hip", "split_hd256_ws4.hip", "kv_append.hip", "stream_read.hip")
+           "split_hd256_ws.hip", "split_hd256_ws4.hip", "split_hd64_wide.hip",
+           "split_hd128_wide.hip", "kv_append.hip", "stream_read.hip")
 # Comparison build: QK always on the matrix cores (the default build puts it on
 # the VALU for launches of few columns at head dims >= 128).
 QK_MFMA_LIB_PATH = PACKAGE_DIR / "_lib" / "qk_mfma" / "libmxfa_mi355x.so"
@@ -165,6 +166,7 @@ def torch_op_command(output: Path) -> list[str]:
             "-DTORCH_EXTENSION_NAME=_mxfa_torch", "-DTORCH_API_INCLUDE_EXTENSION_H",
             *[f"-I{p}" for p in cpp_extension.include_paths()],
             f"-I{sysconfig.get_paths()['include']}", f"-I{rocm}/include", f"-I{INCLUDE_DIR}",
+            f"-I{CSRC_DIR}",
             str(TORCH_OP_SOURCE), f"-L{torch_lib}", f"-L{LIB_DIR}", "-lmxfa_mi355x", "-lc10",
             "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python",
             f"-Wl,-rpath,{torch_lib}", "-Wl,-rpath,$ORIGIN", "-o", str(output)]

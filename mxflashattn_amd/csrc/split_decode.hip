@@ -10,6 +10,7 @@
 
 #include <mutex>
 
+#include "mxfa_package.h"
 #include "split_kernels.h"
 
 namespace mxfa {
@@ -62,6 +63,8 @@ int launch_partial_128_ws4(const DecodeParams &p, const Grid &g, int dtype, bool
                            hipStream_t st);
 int launch_partial_256_ws4(const DecodeParams &p, const Grid &g, int dtype, bool fp8,
                            hipStream_t st);
+int launch_wide_64(const DecodeParams &p, const Grid &g, int dtype, bool fp8, hipStream_t st);
+int launch_wide_128(const DecodeParams &p, const Grid &g, int dtype, bool fp8, hipStream_t st);
 int launch_combine_64(const CombineParams &c, int dtype, hipStream_t st);
 int launch_combine_128(const CombineParams &c, int dtype, hipStream_t st);
 int launch_combine_256(const CombineParams &c, int dtype, hipStream_t st);
@@ -134,6 +137,7 @@ struct SplitArgs {
   float softcap;       // logit soft-capping (0: none)
   const float *alibi;  // per query head ALiBi slopes, nullptr: none
   int min_seqlen_add;  // 0, or -2^30 where lengths below zero count as 0
+  int max_cols;        // columns (query tokens x heads per kv head) the entry point takes
 };
 
 struct WsLayout {
@@ -164,7 +168,7 @@ static int check_call_args(const SplitArgs &a) {
   if (a.ql <= 0 || a.window_left < -1) return MXFA_EINVAL;
   if (!(a.softcap >= 0.f) || a.softcap == INFINITY) return MXFA_EINVAL;
   if (a.window_left > (1 << 30)) return MXFA_EUNSUPPORTED;
-  if (gq * a.ql > kMaxCols) return MXFA_EUNSUPPORTED;
+  if (gq * a.ql > a.max_cols || gq > kMaxCols) return MXFA_EUNSUPPORTED;
   if (a.dtype != MXFA_DTYPE_F16 && a.dtype != MXFA_DTYPE_BF16) return MXFA_EUNSUPPORTED;
   if (ilog2_exact(a.ps) < 0 || a.ps > 4096) return MXFA_EUNSUPPORTED;
   if (a.num_splits > 65535 || a.batch > kMaxBatch || a.hkv > 65535) return MXFA_EUNSUPPORTED;
@@ -270,6 +274,12 @@ static DecodeParams make_params(const SplitArgs &a, const Grid &g) {
 }
 
 static int launch_partial(const SplitArgs &a, hipStream_t st) {
+  if (a.hq / a.hkv * a.ql > kMaxCols) {
+    const Grid g = grid_for(a.hkv, a.num_splits, kMinWaves);
+    const DecodeParams p = make_params(a, g);
+    return a.hd == 64 ? launch_wide_64(p, g, a.dtype, a.fp8, st)
+                      : launch_wide_128(p, g, a.dtype, a.fp8, st);
+  }
   Grid g = grid_for(a.hkv, a.num_splits, waves_for(a.hd * (a.fp8 ? 1 : 2), a.hkv));
   // The host's bound on tiles per range: every sequence at the table's
   // capacity (the lengths are on the device).
@@ -400,6 +410,7 @@ static SplitArgs split_args(const void *q, int64_t q_stride_b, int64_t q_stride_
   a.softcap = 0.f;
   a.alibi = nullptr;
   a.min_seqlen_add = 0;
+  a.max_cols = kMaxCols;
   return a;
 }
 
@@ -468,7 +479,8 @@ static int split_heuristic(int batch, int q_heads, int kv_heads, int head_dim, i
                         (head_dim < 256 || seq_work <= 8192);
   // q_heads / kv_heads columns per launch (q_heads * q_len for the multi-token
   // entry point) must fit the kernel's LDS.
-  const bool fits = seq_lds_bytes(head_dim, (q_heads + kv_heads - 1) / kv_heads) <= kSeqLdsMax;
+  const int cols = (q_heads + kv_heads - 1) / kv_heads;
+  const bool fits = cols <= kMaxCols && seq_lds_bytes(head_dim, cols) <= kSeqLdsMax;
   if (page_size >= kTile && seq_work <= 16384 && fits && (short_rows || mid_rows)) {
     *num_splits = MXFA_SPLITS_PER_SEQUENCE;
     return MXFA_OK;
@@ -476,7 +488,8 @@ static int split_heuristic(int batch, int q_heads, int kv_heads, int head_dim, i
   // One range per wave: one workgroup (waves_for waves) fills every CU, and
   // each wave streams one (kv head, range). The kernel lowers the count to the
   // real tile total on the device.
-  const Grid g = grid_for(kv_heads, 1, waves_for(row_bytes, kv_heads));
+  const Grid g =
+      grid_for(kv_heads, 1, cols > kMaxCols ? kMinWaves : waves_for(row_bytes, kv_heads));
   int64_t n = (int64_t)num_cus * g.subs / g.gx;
   const int64_t cap_tiles = (int64_t)batch * seq_tiles;
   if (n > cap_tiles) n = cap_tiles;
@@ -484,6 +497,29 @@ static int split_heuristic(int batch, int q_heads, int kv_heads, int head_dim, i
   if (n > 65535) n = 65535;
   *num_splits = (int)n;
   return MXFA_OK;
+}
+
+// The general call (several query tokens, window, sinks, cap, ALiBi, fp8
+// caches) as both entry points take it: at most max_cols columns.
+static int run_tokens(SplitArgs a, int64_t q_stride_t, int q_len, int causal, int window_left,
+                      const float *sinks, float softcap, const float *alibi_slopes,
+                      int64_t out_stride_t, int kv_dtype, const float *k_scale,
+                      const float *v_scale, bool wide, hipStream_t st) {
+  if (kv_dtype == MXFA_DTYPE_FP8_E4M3) a = fp8_args(a, k_scale, v_scale);
+  else if (kv_dtype != a.dtype) return MXFA_EUNSUPPORTED;
+  a.q_st = q_stride_t;
+  a.o_st = out_stride_t;
+  a.ql = q_len;
+  a.causal = causal;
+  a.window_left = window_left;
+  a.sinks = sinks;
+  a.softcap = softcap;
+  a.alibi = alibi_slopes;
+  a.min_seqlen_add = -(1 << 30);  // a window on the tokens before the cache end
+  if (wide && a.num_splits > 0)
+    a.max_cols = launch_columns(a.hd, a.ps, a.fp8,
+                                window_left >= 0 || softcap > 0.f || sinks || alibi_slopes);
+  return run_split(a, true, st);
 }
 
 }  // namespace mxfa
@@ -660,23 +696,28 @@ int mxfa_split_decode_multi_launch(
     float scale, int batch, int q_heads, int kv_heads, int head_dim, int page_size,
     int block_table_width, int num_pages, int dtype, int kv_dtype, const float *k_scale,
     const float *v_scale, int num_splits, void *stream) {
-  SplitArgs a = split_args(q, q_stride_b, q_stride_h, k_cache, v_cache, cache_stride_page,
-                           cache_stride_token, cache_stride_head, block_table, bt_stride,
-                           seqlens, seqlen_add, out, out_stride_b, out_stride_h, workspace,
-                           workspace_bytes, scale, batch, q_heads, kv_heads, head_dim, page_size,
-                           block_table_width, num_pages, dtype, num_splits);
-  if (kv_dtype == MXFA_DTYPE_FP8_E4M3) a = fp8_args(a, k_scale, v_scale);
-  else if (kv_dtype != dtype) return MXFA_EUNSUPPORTED;
-  a.q_st = q_stride_t;
-  a.o_st = out_stride_t;
-  a.ql = q_len;
-  a.causal = causal;
-  a.window_left = window_left;
-  a.sinks = sinks;
-  a.softcap = softcap;
-  a.alibi = alibi_slopes;
-  a.min_seqlen_add = -(1 << 30);  // a window on the tokens before the cache end
-  return run_split(a, true, (hipStream_t)stream);
+  return run_tokens(split_args(MXFA_SPLIT_ARGS), q_stride_t, q_len, causal, window_left, sinks,
+                    softcap, alibi_slopes, out_stride_t, kv_dtype, k_scale, v_scale, false,
+                    (hipStream_t)stream);
+}
+
+int mxfa_package_decode_tokens_launch(
+    const void *q, int64_t q_stride_b, int64_t q_stride_t, int64_t q_stride_h, int q_len,
+    int causal, int window_left, const float *sinks, float softcap, const float *alibi_slopes,
+    const void *k_cache, const void *v_cache, int64_t cache_stride_page,
+    int64_t cache_stride_token, int64_t cache_stride_head, const int32_t *block_table,
+    int64_t bt_stride, const int32_t *seqlens, int seqlen_add, void *out, int64_t out_stride_b,
+    int64_t out_stride_t, int64_t out_stride_h, void *workspace, size_t workspace_bytes,
+    float scale, int batch, int q_heads, int kv_heads, int head_dim, int page_size,
+    int block_table_width, int num_pages, int dtype, int kv_dtype, const float *k_scale,
+    const float *v_scale, int num_splits, void *stream) {
+  return run_tokens(split_args(MXFA_SPLIT_ARGS), q_stride_t, q_len, causal, window_left, sinks,
+                    softcap, alibi_slopes, out_stride_t, kv_dtype, k_scale, v_scale, true,
+                    (hipStream_t)stream);
+}
+
+int mxfa_package_launch_columns(int head_dim, int page_size, int fp8, int extras) {
+  return launch_columns(head_dim, page_size, fp8 != 0, extras != 0);
 }
 
 }  // extern "C"

@@ -1,0 +1,12 @@
+// Instantiation unit of the split partial kernel for head dim 64 and more
+// than 16 columns (several query tokens per sequence), two or four groups of
+// 16 columns per wave.
+#include "split_kernels.h"
+
+namespace mxfa {
+
+int launch_wide_64(const DecodeParams &p, const Grid &g, int dtype, bool fp8, hipStream_t st) {
+  return launch_wide_hd<64>(p, g, dtype, fp8, st);
+}
+
+}  // namespace mxfa

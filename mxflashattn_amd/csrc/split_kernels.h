@@ -87,7 +87,7 @@ constexpr float kRescaleLog2 = 8.0f;
 // Tile prefix sums live in LDS, (B + 1) int32 next to a few bytes of static
 // LDS: 16000 sequences keep a workgroup within 64 KB.
 constexpr int kMaxBatch = 16000;
-constexpr int kMaxCols = 16;      // query tokens x heads per kv head: the 16 MFMA columns
+constexpr int kMaxCols = 16;      // query tokens x heads per kv head: the 16 MFMA columns of a group
 constexpr int kOffOut = 0x40000000;          // a lane offset no descriptor covers
 
 // Tile flags.
@@ -770,9 +770,13 @@ struct Tile {
 // kProbe (the streaming probe): the same tile walk and loads, but each tile
 // only XORs the words it loaded into the returned value, with no attention
 // math and no output; other instantiations return 0.
+//
+// kGroups > 1 (HR 4): up to 16 * kGroups columns. Column 16g + c is column c
+// of group g, with its own QK result, softmax state and PV accumulators; the
+// K and V words of a tile are loaded (and widened or paired) once for all.
 template <int HD, int HR, typename T, bool kF8, bool kLanePages, int NBUF, bool kExtras,
           bool kSeq, bool kBalance = false, bool kProbe = false, int kWaveLocal = 0,
-          int kValuG = 0>
+          int kValuG = 0, int kGroups = 1>
 __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32_t *s_tiles,
                                               int kvh, int rr, int lo, int hi, int stride,
                                               float *lds_o, float *lds_lse, int pg_first = 0,
@@ -832,18 +836,22 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
   // last c_hide keys of the sequence from it, and the window all keys more
   // than c_reach from the sequence end. Key k of a sequence of L keys is seen
   // when c_hide < L - k <= c_reach.
-  const int ct = col / gq, cg = col - (col / gq) * gq;
-  const int c_hide = p.causal ? p.ql - 1 - ct : 0;
-  const int c_reach = p.window_left >= 0 ? p.ql - ct + p.window_left : 0x3fffffff;
+  int c_hide[kGroups], c_reach[kGroups], qdist[kGroups], q_off[kGroups];
+  float slope2[kGroups];
   // ALiBi: base-2 slope of this lane's column; the query of column (ct, cg)
   // sits QL - ct keys before the sequence end, so key k (L - k = rel) is
   // |rel - (QL - ct)| positions away from it.
   const bool alibi = kExtras && p.alibi != nullptr;
-  const float slope2 =
-      alibi && col < nc ? ((ConstF32)p.alibi)[kvh * gq + cg] * kLog2e : 0.f;
-  const int qdist = p.ql - ct;
-  const int q_off =
-      col < nc ? ct * (int)p.q_st + cg * (int)p.q_sh + row * (kF8 ? 32 : 16) : kOffOut;
+#pragma unroll
+  for (int g = 0; g < kGroups; ++g) {
+    const int cl = 16 * g + col;
+    const int ct = cl / gq, cg = cl - (cl / gq) * gq;
+    c_hide[g] = p.causal ? p.ql - 1 - ct : 0;
+    c_reach[g] = p.window_left >= 0 ? p.ql - ct + p.window_left : 0x3fffffff;
+    slope2[g] = alibi && cl < nc ? ((ConstF32)p.alibi)[kvh * gq + cg] * kLog2e : 0.f;
+    qdist[g] = p.ql - ct;
+    q_off[g] = cl < nc ? ct * (int)p.q_st + cg * (int)p.q_sh + row * (kF8 ? 32 : 16) : kOffOut;
+  }
   const int q_bytes = (p.ql - 1) * (int)p.q_st + (gq - 1) * (int)p.q_sh + HD * 2;
   auto q_step = [](int cc) { return kF8 ? (cc >> 1) * 128 + (cc & 1) * 16 : cc * 64; };
 
@@ -984,7 +992,7 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
     uint4 k[NKL];
     Frag<VB> v[kShareV ? 1 : U];  // kShareV: unused
     uint4 vr[kShareV ? 2 : 1];    // kShareV: tokens 4r+2h, 4r+2h+1, 16 bytes each
-    uint4 q[NCH];
+    uint4 q[kGroups][NCH];
     int lpg[NPG];
     Tile d;
   };
@@ -998,7 +1006,9 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
                  rfl((d.flags & kFirst) ? q_bytes : 0));
     if (d.flags & kFirst) {  // wave-uniform; q is loaded once per piece
 #pragma unroll
-      for (int cc = 0; cc < NCH; ++cc) s.q[cc] = buf_load16<0>(rq, q_off + q_step(cc));
+      for (int g = 0; g < kGroups; ++g)
+#pragma unroll
+        for (int cc = 0; cc < NCH; ++cc) s.q[g][cc] = buf_load16<0>(rq, q_off[g] + q_step(cc));
     }
     if constexpr (!kLanePages) {
       const uint64_t tile_off = (uint64_t)(uint32_t)clamp_page(d.pg) * (uint64_t)p.sp_bytes +
@@ -1039,18 +1049,25 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
   };
 
   // Running state of the current piece.
-  float m = -INFINITY;  // reference max (base 2) of column `col`, same in every row
-  float dsum = 0.f;     // partial denominator of column `col` over this row's tokens
-  f32x4 oacc[VD];       // PV accumulators
-  uint4 qf[NCH];
+  float m[kGroups];           // reference max (base 2) of column `col`, same in every row
+  float dsum[kGroups];        // partial denominator of column `col` over this row's tokens
+  f32x4 oacc[kGroups][VD];    // PV accumulators
+  uint4 qf[kGroups][NCH];
   uint4 qv[kValu ? kValuG : 1][NCH];  // kValu: column g's chunk c%4 of each step, lane (r, c)
   auto clear_acc = [&]() {
 #pragma unroll
-    for (int j = 0; j < VD; ++j) oacc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int g = 0; g < kGroups; ++g) {
+      m[g] = -INFINITY;
+      dsum[g] = 0.f;
+#pragma unroll
+      for (int j = 0; j < VD; ++j) oacc[g][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
   };
   clear_acc();
 #pragma unroll
-  for (int cc = 0; cc < NCH; ++cc) qf[cc] = make_uint4(0u, 0u, 0u, 0u);
+  for (int g = 0; g < kGroups; ++g)
+#pragma unroll
+    for (int cc = 0; cc < NCH; ++cc) qf[g][cc] = make_uint4(0u, 0u, 0u, 0u);
   bool piece_from_start = false;
   bool piece_first_in_range = false;
 #ifdef MXFA_WAVE_STAMPS
@@ -1060,43 +1077,46 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
   const int vslot = kShareV ? 2 * (col & 7) + (col >> 3) : col;
 
   auto finalize = [&](const Tile &d) {
-    const float dt = rows_sum(dsum);  // lane (any row, h): denominator of head h
     const int b = d.b;
     const bool whole = !kSeq && piece_from_start && (d.flags & kSeqEnd);
     const int slot = piece_first_in_range ? 0 : 1;
     const int64_t pbase = ((int64_t)(kvh * ns + rr) * 2 + slot) * nc;
-    static_for<4>([&](auto ic) {
-      constexpr int i = decltype(ic)::value;
-      const int hh = 4 * row + i;  // column of accumulator element i in this lane
-      const float Dh = head_of_row<HR, i>(dt, row);
-      const float Mh = head_of_row<HR, i>(m, row);
-      if (hh >= nc) return;
-      const int ht = hh / gq, hg = hh - (hh / gq) * gq;
-      // A sink joins the denominator once per (sequence, head): here for a
-      // sequence whole in the range, in the combine for a split one. With no
-      // key seen (Mh = -inf) the term is +inf and the output 0.
-      float Dw = Dh;
-      if constexpr (kExtras) {
-        if (whole && p.sinks) Dw += fast_exp2(p.sinks[kvh * gq + hg] * kLog2e - Mh);
-      }
-      const float inv = Dw > 0.f ? v_scale / Dw : 0.f;
-      float v[VD];
+    static_for<kGroups>([&](auto gc) {
+      constexpr int g = decltype(gc)::value;
+      const float dt = rows_sum(dsum[g]);  // lane (any row, h): denominator of head h
+      static_for<4>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        const int hh = 16 * g + 4 * row + i;  // column of accumulator element i in this lane
+        const float Dh = head_of_row<HR, i>(dt, row);
+        const float Mh = head_of_row<HR, i>(m[g], row);
+        if (hh >= nc) return;
+        const int ht = hh / gq, hg = hh - (hh / gq) * gq;
+        // A sink joins the denominator once per (sequence, head): here for a
+        // sequence whole in the range, in the combine for a split one. With no
+        // key seen (Mh = -inf) the term is +inf and the output 0.
+        float Dw = Dh;
+        if constexpr (kExtras) {
+          if (whole && p.sinks) Dw += fast_exp2(p.sinks[kvh * gq + hg] * kLog2e - Mh);
+        }
+        const float inv = Dw > 0.f ? v_scale / Dw : 0.f;
+        float v[VD];
 #pragma unroll
-      for (int j = 0; j < VD; ++j) v[j] = oacc[j][i];
-      if (whole) {
-        store_row<VD, E>(p.out + b * p.o_sb + ht * p.o_st + (kvh * gq + hg) * p.o_sh +
-                             vslot * (VD * 2),
-                         v, inv);
-      } else {
-        float4 *dst = reinterpret_cast<float4 *>(
-            (kSeq ? lds_o + hh * HD : p.ws_o + (pbase + hh) * HD) + vslot * VD);
+        for (int j = 0; j < VD; ++j) v[j] = oacc[g][j][i];
+        if (whole) {
+          store_row<VD, E>(p.out + b * p.o_sb + ht * p.o_st + (kvh * gq + hg) * p.o_sh +
+                               vslot * (VD * 2),
+                           v, inv);
+        } else {
+          float4 *dst = reinterpret_cast<float4 *>(
+              (kSeq ? lds_o + hh * HD : p.ws_o + (pbase + hh) * HD) + vslot * VD);
 #pragma unroll
-        for (int j = 0; j < VD / 4; ++j)
-          dst[j] = make_float4(v[4 * j] * inv, v[4 * j + 1] * inv, v[4 * j + 2] * inv,
-                               v[4 * j + 3] * inv);
-        if (col == 0)
-          (kSeq ? lds_lse[hh] : p.ws_lse[pbase + hh]) = Dh > 0.f ? Mh + __log2f(Dh) : -INFINITY;
-      }
+          for (int j = 0; j < VD / 4; ++j)
+            dst[j] = make_float4(v[4 * j] * inv, v[4 * j + 1] * inv, v[4 * j + 2] * inv,
+                                 v[4 * j + 3] * inv);
+          if (col == 0)
+            (kSeq ? lds_lse[hh] : p.ws_lse[pbase + hh]) = Dh > 0.f ? Mh + __log2f(Dh) : -INFINITY;
+        }
+      });
     });
   };
 
@@ -1117,16 +1137,17 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
       }
       if (d.flags & kFirst) {
 #pragma unroll
-        for (int cc = 0; cc < NCH; ++cc) probe ^= s.q[cc].x ^ s.q[cc].y ^ s.q[cc].z ^ s.q[cc].w;
+        for (int cc = 0; cc < NCH; ++cc)
+          probe ^= s.q[0][cc].x ^ s.q[0][cc].y ^ s.q[0][cc].z ^ s.q[0][cc].w;
       }
       return;
     }
     if (d.flags & kFirst) {
-      m = -INFINITY;
-      dsum = 0.f;
       clear_acc();
 #pragma unroll
-      for (int cc = 0; cc < NCH; ++cc) qf[cc] = s.q[cc];
+      for (int g = 0; g < kGroups; ++g)
+#pragma unroll
+        for (int cc = 0; cc < NCH; ++cc) qf[g][cc] = s.q[g][cc];
       if constexpr (kValu) {
         // qf: lane (r', c') holds column c' chunk r'; column g chunk k sits in
         // lane 16k + g (the LDS crossbar moves it; no LDS memory is used).
@@ -1135,10 +1156,10 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
           const int src = ((col & 3) * 16 + g) * 4;
 #pragma unroll
           for (int cc = 0; cc < NCH; ++cc) {
-            qv[g][cc].x = __builtin_amdgcn_ds_bpermute(src, qf[cc].x);
-            qv[g][cc].y = __builtin_amdgcn_ds_bpermute(src, qf[cc].y);
-            qv[g][cc].z = __builtin_amdgcn_ds_bpermute(src, qf[cc].z);
-            qv[g][cc].w = __builtin_amdgcn_ds_bpermute(src, qf[cc].w);
+            qv[g][cc].x = __builtin_amdgcn_ds_bpermute(src, qf[0][cc].x);
+            qv[g][cc].y = __builtin_amdgcn_ds_bpermute(src, qf[0][cc].y);
+            qv[g][cc].z = __builtin_amdgcn_ds_bpermute(src, qf[0][cc].z);
+            qv[g][cc].w = __builtin_amdgcn_ds_bpermute(src, qf[0][cc].w);
           }
         }
       }
@@ -1146,7 +1167,9 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
       piece_first_in_range = (d.flags & kRangeStart) != 0;
     }
     // QK on the matrix cores; two accumulators halve the MFMA dependency chain.
-    f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+    f32x4 acc0[kGroups], acc1[kGroups];
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g) acc0[g] = acc1[g] = f32x4{0.f, 0.f, 0.f, 0.f};
     if constexpr (kValu) {
       // QK on the VALU: per column g, the lane's 4 * NCH dot2 over its chunks
       // of its token, summed over the four chunk lanes of the token (quad_perm
@@ -1179,96 +1202,108 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
           const float b = row_bcast<4 * i>(sg[g]);
           v = col == g ? b : v;
         }
-        acc0[i] = v;
+        acc0[0][i] = v;
       });
     } else if constexpr (kF8) {
 #pragma unroll
       for (int mm = 0; mm < NKL; ++mm) {
-        acc0 = Mfma<T>::run(widen8<T>(s.k[mm].x, s.k[mm].y), qf[2 * mm], acc0);
-        acc1 = Mfma<T>::run(widen8<T>(s.k[mm].z, s.k[mm].w), qf[2 * mm + 1], acc1);
+        const uint4 ka = widen8<T>(s.k[mm].x, s.k[mm].y), kb = widen8<T>(s.k[mm].z, s.k[mm].w);
+#pragma unroll
+        for (int g = 0; g < kGroups; ++g) {
+          acc0[g] = Mfma<T>::run(ka, qf[g][2 * mm], acc0[g]);
+          acc1[g] = Mfma<T>::run(kb, qf[g][2 * mm + 1], acc1[g]);
+        }
       }
     } else {
 #pragma unroll
       for (int cc = 0; cc < NCH; cc += 2) {
-        acc0 = Mfma<T>::run(s.k[cc], qf[cc], acc0);
-        acc1 = Mfma<T>::run(s.k[cc + 1], qf[cc + 1], acc1);
-      }
-    }
-    float x[4];
-    bool need = false;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = (acc0[i] + acc1[i]) * c;
-    if constexpr (kExtras) {
-      if (capped) {  // wave-uniform
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x[i] = cap_out * tanh_exp2((acc0[i] + acc1[i]) * cap_in);
-      }
-      if (alibi) {  // wave-uniform; after the cap, as FlashAttention applies it
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int dist = abs(d.rem - (4 * row + i) - qdist);
-          x[i] -= slope2 * (float)dist;
+        for (int g = 0; g < kGroups; ++g) {
+          acc0[g] = Mfma<T>::run(s.k[cc], qf[g][cc], acc0[g]);
+          acc1[g] = Mfma<T>::run(s.k[cc + 1], qf[g][cc + 1], acc1[g]);
         }
       }
     }
+    uint2 a[kGroups];  // P of each group, packed pairs of the element type
+    static_for<kGroups>([&](auto gc) {
+      constexpr int g = decltype(gc)::value;
+      float x[4];
+      bool need = false;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = 4 * row + i;
-      bool valid = (col < nc) & (r < d.rem - c_hide);
-      if constexpr (kExtras) valid &= r >= d.rem - c_reach;
-      x[i] = valid ? x[i] : -INFINITY;
-      need |= x[i] > m + kRescaleLog2;
-    }
+      for (int i = 0; i < 4; ++i) x[i] = (acc0[g][i] + acc1[g][i]) * c;
+      if constexpr (kExtras) {
+        if (capped) {  // wave-uniform
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            x[i] = cap_out * tanh_exp2((acc0[g][i] + acc1[g][i]) * cap_in);
+        }
+        if (alibi) {  // wave-uniform; after the cap, as FlashAttention applies it
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int dist = abs(d.rem - (4 * row + i) - qdist[g]);
+            x[i] -= slope2[g] * (float)dist;
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 4 * row + i;
+        bool valid = (16 * g + col < nc) & (r < d.rem - c_hide[g]);
+        if constexpr (kExtras) valid &= r >= d.rem - c_reach[g];
+        x[i] = valid ? x[i] : -INFINITY;
+        need |= x[i] > m[g] + kRescaleLog2;
+      }
 #ifdef MXFA_WAVE_STAMPS
-    if (stamp_data) {
-      wave_stamp_after(p, 11, x[0]);
-      stamp_data = false;
-    }
+      if (stamp_data) {
+        wave_stamp_after(p, 11, x[0]);
+        stamp_data = false;
+      }
 #endif
-    if (__builtin_amdgcn_ballot_w64(need) != 0) {
-      // Rare, wave-uniform: move the reference of each head to the wave's
-      // tile maximum when it passed the reference by more than kRescaleLog2.
-      const float mt = rows_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
-      const float mn = mt > m + kRescaleLog2 ? mt : m;
-      const float f = (mn == m) ? 1.f : fast_exp2(m - mn);  // m = -inf: f = 0
-      dsum *= f;
-      static_for<4>([&](auto ic) {
-        constexpr int i = decltype(ic)::value;
-        const float fi = head_of_row<HR, i>(f, row);
+      if (__builtin_amdgcn_ballot_w64(need) != 0) {
+        // Rare, wave-uniform: move the reference of each head to the wave's
+        // tile maximum when it passed the reference by more than kRescaleLog2.
+        const float mt = rows_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
+        const float mn = mt > m[g] + kRescaleLog2 ? mt : m[g];
+        const float f = (mn == m[g]) ? 1.f : fast_exp2(m[g] - mn);  // m = -inf: f = 0
+        dsum[g] *= f;
+        static_for<4>([&](auto ic) {
+          constexpr int i = decltype(ic)::value;
+          const float fi = head_of_row<HR, i>(f, row);
 #pragma unroll
-        for (int j = 0; j < VD; ++j) oacc[j][i] *= fi;
-      });
-      m = mn;
-    }
-    // m = -inf: this column has seen no valid token, its scores here are -inf too.
-    const float mr = m == -INFINITY ? 0.f : m;
-    float pr[4];
+          for (int j = 0; j < VD; ++j) oacc[g][j][i] *= fi;
+        });
+        m[g] = mn;
+      }
+      // m = -inf: this column has seen no valid token, its scores here are -inf too.
+      const float mr = m[g] == -INFINITY ? 0.f : m[g];
+      float pr[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) pr[i] = fast_exp2(x[i] - mr);
-    // P rounded to the element type once; the denominator sums the same
-    // rounded weights, so the output stays a convex combination of V rows.
-    uint16_t ph[4];
+      for (int i = 0; i < 4; ++i) pr[i] = fast_exp2(x[i] - mr);
+      // P rounded to the element type once; the denominator sums the same
+      // rounded weights, so the output stays a convex combination of V rows.
+      uint16_t ph[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) ph[i] = PvMfma<T>::round(pr[i]);
-    dsum += (PvMfma<T>::widen(ph[0]) + PvMfma<T>::widen(ph[1])) +
-            (PvMfma<T>::widen(ph[2]) + PvMfma<T>::widen(ph[3]));
-    const uint2 a = make_uint2((uint32_t)ph[0] | ((uint32_t)ph[1] << 16),
-                               (uint32_t)ph[2] | ((uint32_t)ph[3] << 16));
+      for (int i = 0; i < 4; ++i) ph[i] = PvMfma<T>::round(pr[i]);
+      dsum[g] += (PvMfma<T>::widen(ph[0]) + PvMfma<T>::widen(ph[1])) +
+                 (PvMfma<T>::widen(ph[2]) + PvMfma<T>::widen(ph[3]));
+      a[g] = make_uint2((uint32_t)ph[0] | ((uint32_t)ph[1] << 16),
+                        (uint32_t)ph[2] | ((uint32_t)ph[3] << 16));
+    });
     // The lane's V bytes of its four tokens (kShareV: halves swapped with lane
     // c^8 first), then as element pairs (fp8: widened here, once).
     constexpr int VW = VB / 4;  // words per token
     uint32_t vt[U][VW];
     if constexpr (kShareV) {
       const bool hi = col >= 8;
-      const uint4 a = s.vr[0], bq = s.vr[1];
-      const uint32_t r0 = row_swap8(hi ? a.x : a.z), r1 = row_swap8(hi ? a.y : a.w);
+      const uint4 va = s.vr[0], bq = s.vr[1];
+      const uint32_t r0 = row_swap8(hi ? va.x : va.z), r1 = row_swap8(hi ? va.y : va.w);
       const uint32_t r2 = row_swap8(hi ? bq.x : bq.z), r3 = row_swap8(hi ? bq.y : bq.w);
-      vt[0][0] = hi ? r0 : a.x;
-      vt[0][1] = hi ? r1 : a.y;
+      vt[0][0] = hi ? r0 : va.x;
+      vt[0][1] = hi ? r1 : va.y;
       vt[1][0] = hi ? r2 : bq.x;
       vt[1][1] = hi ? r3 : bq.y;
-      vt[2][0] = hi ? a.z : r0;
-      vt[2][1] = hi ? a.w : r1;
+      vt[2][0] = hi ? va.z : r0;
+      vt[2][1] = hi ? va.w : r1;
       vt[3][0] = hi ? bq.z : r2;
       vt[3][1] = hi ? bq.w : r3;
     } else {
@@ -1294,7 +1329,8 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
       const int wi = jb >> 1, odd = jb & 1;
       const uint2 bv = make_uint2(pair_halves(vw[0][wi], vw[1][wi], odd),
                                   pair_halves(vw[2][wi], vw[3][wi], odd));
-      oacc[jb] = PvMfma<T>::run(a, bv, oacc[jb]);
+#pragma unroll
+      for (int g = 0; g < kGroups; ++g) oacc[g][jb] = PvMfma<T>::run(a[g], bv, oacc[g][jb]);
     }
     if (d.flags & kLast) finalize(d);
   };
@@ -1366,7 +1402,7 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
 // kExtras: the call has a sliding window, soft-capping, ALiBi or sinks (the host
 // picks the instantiation; without them the kernel is the plain one).
 template <int HD, int HR, typename T, bool kF8, bool kLanePages, int NBUF, int WAVES,
-          bool kExtras, int kWaveScan, int kValuG>
+          bool kExtras, int kWaveScan, int kValuG, int kGroups = 1>
 __global__ __launch_bounds__(WAVES * 64, 1) void split_partial_kernel(const int32_t *seqlens,
                                                                         int batch,
                                                                         DecodeParams p) {
@@ -1402,7 +1438,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void split_partial_kernel(const int3
   wave_stamp(p, 0, t_entry);
   wave_stamp(p, 1, wave_clock());
   run_range<HD, HR, T, kF8, kLanePages, NBUF, kExtras, false, WAVES == 8, false, kWaveScan,
-            kValuG>(p, s_tiles, kvh, rr, lo, hi, 1, nullptr, nullptr, 0, wsc);
+            kValuG, kGroups>(p, s_tiles, kvh, rr, lo, hi, 1, nullptr, nullptr, 0, wsc);
   // The prefix sums for the combine, by the first wave of workgroup (0, 0)
   // (which always has a range) once its own range is done: the pointer is
   // read from the parameter block only here, off the prologue.
@@ -1706,6 +1742,10 @@ inline Grid grid_for(int hkv, int num_splits, int waves) {
 template <int HD, bool kF8>
 constexpr int kNbuf = kRowBytes<HD, kF8> <= 64 ? 4 : kRowBytes<HD, kF8> <= 128 ? 3 : 2;
 
+// Register sets of launches of more than 16 columns (several groups per wave).
+template <int HD, bool kF8>
+constexpr int kWideNbuf = kNbuf<HD, kF8>;
+
 // Eight-wave workgroups of 128-byte rows (two waves per SIMD) take two
 // register sets instead of three when the host's bound on tiles per range is
 // small: the shorter pipeline fill and drain pay more than the third set's
@@ -1845,6 +1885,71 @@ int launch_partial_hd(const DecodeParams &p, const Grid &g, int dtype, bool fp8,
                : launch_partial_hr<HD, BF16, false, kWaveScan>(p, g, st);
   return fp8 ? launch_partial_hr<HD, F16, true, kWaveScan>(p, g, st)
              : launch_partial_hr<HD, F16, false, kWaveScan>(p, g, st);
+}
+
+// More than 16 columns (several query tokens): kGroups groups of 16 columns
+// per wave, so the keys are read once for all of them. One wave per SIMD
+// (four-wave workgroups), so that a wave has 512 registers, and as many groups
+// as fit them without a spill: four at head dim 64; three at head dim 128 (96
+// registers in PV accumulators, 144 in q), two of them with a window, cap,
+// sinks or ALiBi; two with fp8 caches (a third register set and the widened
+// operands); one at head dim 256.
+// Measured on MI355X against launches of 16 columns that each read the keys
+// again (graph replays, B 32, 8 kv heads, GQ 4, bf16, L ~ U[2048, 4096], us per
+// call): head dim 128, 5 tokens 141.4 -> 80.4, 8 tokens 154.2 -> 85.0, 12 tokens
+// 228.8 -> 94.8, 16 tokens (two launches instead of four) 296.5 -> 167.2; head
+// dim 64, 8 tokens 90.7 -> 50.8, 16 tokens 174.5 -> 75.4. One pass over the
+// keys is bound by HBM up to 32 columns at head dim 128 (85 us against 79 for
+// one token); past that, and at head dim 64, each group's softmax and matrix
+// instructions show, since one wave per SIMD has nothing to hide them behind.
+template <int HD, bool kF8, bool kExtras>
+constexpr int kMostGroups = HD > 128 ? 1 : kF8 ? 2 : HD == 64 ? 4 : kExtras ? 2 : 3;
+
+// Columns one launch takes: page-uniform tiles (page size >= 16), else 16.
+inline int launch_columns(int hd, int ps, bool fp8, bool extras) {
+  if (ps < kTile || hd > 128) return kMaxCols;
+  if (hd == 64) return 16 * (fp8 ? kMostGroups<64, true, false> : kMostGroups<64, false, false>);
+  return 16 * (fp8      ? kMostGroups<128, true, false>
+               : extras ? kMostGroups<128, false, true>
+                        : kMostGroups<128, false, false>);
+}
+
+template <int HD, typename T, bool kF8, bool kExtras, int kWaveScan, int kGroups>
+static int launch_wide_g(const DecodeParams &p, const Grid &g, hipStream_t st) {
+  const size_t lds = kWaveScan ? 0 : (size_t)(p.batch + 1) * sizeof(int32_t);
+  hipLaunchKernelGGL((split_partial_kernel<HD, 4, T, kF8, false, kWideNbuf<HD, kF8>, 4, kExtras,
+                                           kWaveScan, 0, kGroups>),
+                     dim3(g.gx, g.gy), dim3(256), lds, st, p.seqlens, p.batch, p);
+  return hipGetLastError() == hipSuccess ? MXFA_OK : MXFA_ELAUNCH;
+}
+
+template <int HD, typename T, bool kF8, bool kExtras, int kWaveScan>
+static int launch_wide_s(const DecodeParams &p, const Grid &g, hipStream_t st) {
+  constexpr int kMost = kMostGroups<HD, kF8, kExtras>;
+  if constexpr (kMost > 2) {
+    if (p.gq * p.ql > 32) return launch_wide_g<HD, T, kF8, kExtras, kWaveScan, kMost>(p, g, st);
+  }
+  return launch_wide_g<HD, T, kF8, kExtras, kWaveScan, 2>(p, g, st);
+}
+
+// Plain calls of up to kWaveScanMax1 sequences scan the tiles inside each
+// wave; the others take the LDS scan (fewer instantiations).
+template <int HD, typename T, bool kF8>
+static int launch_wide_x(const DecodeParams &p, const Grid &g, hipStream_t st) {
+  if (!plain_call(p)) return launch_wide_s<HD, T, kF8, true, 0>(p, g, st);
+  if (wave_scan_per_lane(p.batch) == 1) return launch_wide_s<HD, T, kF8, false, 1>(p, g, st);
+  return launch_wide_s<HD, T, kF8, false, 0>(p, g, st);
+}
+
+// Partial kernel of a launch of 17 .. launch_columns columns and a four-wave grid.
+template <int HD>
+int launch_wide_hd(const DecodeParams &p, const Grid &g, int dtype, bool fp8, hipStream_t st) {
+  if (g.waves != 4 || g.heads_per_wg * g.subs > 4 ||
+      p.gq * p.ql > launch_columns(HD, 1 << p.ps_log2, fp8, !plain_call(p)))
+    return MXFA_ELAUNCH;
+  if (dtype == MXFA_DTYPE_BF16)
+    return fp8 ? launch_wide_x<HD, BF16, true>(p, g, st) : launch_wide_x<HD, BF16, false>(p, g, st);
+  return fp8 ? launch_wide_x<HD, F16, true>(p, g, st) : launch_wide_x<HD, F16, false>(p, g, st);
 }
 
 // Per-sequence kernel (seq_decode_kernel): grid (ceil(HKV / KH), B) of

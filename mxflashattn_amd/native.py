@@ -61,8 +61,10 @@ SUPPORTED_GQA = (2, 4, 8)
 KERNEL_HEAD_DIMS = (64, 128, 256)
 KERNEL_GQA = tuple(range(1, 17))
 KERNEL_COLUMNS = 16
-# Query tokens x GQ that the routing layers send here for a causal query: at
-# most four launches of token chunks, each reading its sequences' keys again.
+# Query tokens x GQ that the routing layers send here for a causal query: one
+# or two launches of several column groups where the kernel has them
+# (launch_columns), else up to four launches of token chunks, each reading its
+# sequences' keys again.
 CHUNKED_COLUMNS = 4 * KERNEL_COLUMNS
 
 # Every entry point declared in include/mxfa_mi355x.h.
@@ -146,6 +148,12 @@ _SIGNATURES = {
     ),
 }
 
+# Entry points for this package only (csrc/mxfa_package.h), not part of the C ABI.
+_PACKAGE_SIGNATURES = {
+    "mxfa_package_launch_columns": (_i, [_i, _i, _i, _i]),
+    "mxfa_package_decode_tokens_launch": _SIGNATURES["mxfa_split_decode_multi_launch"],
+}
+
 _load_lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
 _load_error: str | None = None
@@ -170,7 +178,7 @@ def library() -> ctypes.CDLL:
         except OSError as exc:
             _load_error = f"native library failed to load: {exc}"
             raise NativeLibraryError(_load_error) from exc
-        for name, (restype, argtypes) in _SIGNATURES.items():
+        for name, (restype, argtypes) in (*_SIGNATURES.items(), *_PACKAGE_SIGNATURES.items()):
             fn = getattr(lib, name)
             fn.restype = restype
             fn.argtypes = argtypes
@@ -556,7 +564,7 @@ def _launch_multi(q, k_cache, v_cache, block_table, cache_seqlens, out, workspac
     pages, ps, hkv = k_cache.shape[0], k_cache.shape[1], k_cache.shape[2]
     qs, os_, cs = q.stride(), out.stride(), k_cache.stride()
     fp8 = k_cache.dtype == FP8_DTYPE
-    rc = library().mxfa_split_decode_multi_launch(
+    rc = library().mxfa_package_decode_tokens_launch(
         q.data_ptr(), qs[0], qs[1], qs[2], ql, int(bool(causal)), int(window_left),
         _sinks_ptr(sinks, q), float(softcap), _sinks_ptr(alibi_slopes, q, "alibi_slopes"),
         k_cache.data_ptr(),
@@ -567,6 +575,23 @@ def _launch_multi(q, k_cache, v_cache, block_table, cache_seqlens, out, workspac
         _scale_ptr(k_scale, q.device, "k_scale") if fp8 else 0,
         _scale_ptr(v_scale, q.device, "v_scale") if fp8 else 0, num_splits, stream)
     _check(rc, "mxfa_split_decode_multi_launch")
+
+
+@functools.lru_cache(maxsize=64)
+def launch_columns(head_dim: int, page_size: int, fp8: bool, extras: bool) -> int:
+    """Query tokens x GQ that one split launch takes (16, or more where the
+    kernel keeps several groups of 16 columns and reads the keys once for all)."""
+    return library().mxfa_package_launch_columns(head_dim, page_size, int(fp8), int(extras))
+
+
+def tokens_per_launch(q_len: int, gq: int, columns: int) -> int:
+    """Query tokens of each launch: as many as ``columns`` hold, or, of launches
+    of several column groups, about equal shares (64 columns at head dim 128
+    are two launches of two groups rather than one of three and one of one)."""
+    if columns <= KERNEL_COLUMNS:
+        return min(q_len, columns // gq)
+    launches = -(-q_len // (columns // gq))
+    return -(-q_len // launches)
 
 
 def _sinks_ptr(values, q: torch.Tensor, name: str = "sinks") -> int:
@@ -585,14 +610,24 @@ def _sinks_ptr(values, q: torch.Tensor, name: str = "sinks") -> int:
 def default_num_splits(q: torch.Tensor, k_cache: torch.Tensor, block_table: torch.Tensor) -> int:
     """The heuristic's count for q ([B, HQ, HD] or [B, QL, HQ, HD]). It is
     asked for the columns of one launch, HQ times the query tokens a launch
-    takes (QL, or 16 / GQ of them for longer causal queries), which decide
-    whether the per-sequence kernel's LDS holds them."""
+    takes (QL, or for longer causal queries 16 / GQ of them), which decide
+    whether the per-sequence kernel's LDS holds them; a causal query past 16
+    columns that it gives to the split kernel asks again for the columns that
+    kernel takes at once."""
     hq, hkv = q.shape[-2], k_cache.shape[2]
+    gq = max(1, hq // hkv)
     ql = q.shape[1] if q.dim() == 4 else 1
-    tokens = min(ql, max(1, KERNEL_COLUMNS // max(1, hq // hkv)))
-    return split_heuristic(q.shape[0], hq * tokens, hkv, q.shape[-1], k_cache.shape[1],
-                           block_table.shape[1], num_cus(q.device.index or 0),
-                           k_cache.dtype == FP8_DTYPE)
+    fp8 = k_cache.dtype == FP8_DTYPE
+    batch, hd, ps, width = q.shape[0], q.shape[-1], k_cache.shape[1], block_table.shape[1]
+    cus = num_cus(q.device.index or 0)
+    tokens = min(ql, max(1, KERNEL_COLUMNS // gq))
+    ns = split_heuristic(batch, hq * tokens, hkv, hd, ps, width, cus, fp8)
+    if ql > tokens and ns != SPLITS_PER_SEQUENCE:
+        columns = launch_columns(hd, ps, fp8, False)
+        if columns > KERNEL_COLUMNS:
+            ns = split_heuristic(batch, hq * tokens_per_launch(ql, gq, columns), hkv, hd, ps,
+                                 width, cus, fp8)
+    return ns
 
 
 def paged_decode_split(
@@ -618,8 +653,8 @@ def paged_decode_split(
 
     q: [B, QL, HQ, HD] or [B, HQ, HD] (any strides with a contiguous last dim);
     QL > 1 query tokens sit at the last QL positions of each sequence, and
-    ``causal`` masks the keys after each one (QL * HQ/HKV <= 16 per launch; a
-    causal call with more runs as launches of 16 // (HQ/HKV) tokens, each
+    ``causal`` masks the keys after each one (QL * HQ/HKV <= 16, or for a
+    causal call any number: launch_columns of them per launch, each launch
     reading its sequences' keys again);
     caches: [pages, PS, HKV, HD] of q's dtype, or float8_e4m3fn with the
     per-tensor dequantisation scales k_scale / v_scale (float32 device scalars
@@ -669,13 +704,17 @@ def paged_decode_split(
         num_splits = default_num_splits(q, k_cache, block_table)
     stream = _stream_handle(q.device)
     ql = q.shape[1] if q.dim() == 4 else 1
-    per_launch = KERNEL_COLUMNS // (q.shape[-2] // k_cache.shape[2])
-    ws_bytes = workspace_size(q.shape[0], q.shape[-2] * min(ql, per_launch), q.shape[-1],
-                              num_splits)
+    extras = window_left >= 0 or sinks is not None or softcap > 0 or alibi_slopes is not None
+    gq = q.shape[-2] // k_cache.shape[2]
+    columns = KERNEL_COLUMNS
+    if ql * gq > columns and num_splits != SPLITS_PER_SEQUENCE:
+        columns = launch_columns(q.shape[-1], k_cache.shape[1], k_cache.dtype == FP8_DTYPE,
+                                 extras)
+    per_launch = tokens_per_launch(ql, gq, columns)
+    ws_bytes = workspace_size(q.shape[0], q.shape[-2] * per_launch, q.shape[-1], num_splits)
     ws = WORKSPACE.get(q.device, stream, ws_bytes)
     _poison(out)
-    if ql > 1 or window_left >= 0 or sinks is not None or softcap > 0 or (
-            alibi_slopes is not None):
+    if ql > 1 or extras:
         for first, end, add in token_chunks(ql, per_launch, int(seqlen_add)):
             whole = first == 0 and end == ql
             _poison(None, ws)

@@ -1,0 +1,80 @@
+"""Causal queries of more than 16 columns (query tokens x heads per kv head) in
+one launch: two to four groups of 16 columns per wave, against the reference
+port, at the edges of the groups and of the columns one launch takes."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from mxflashattn_amd import native
+from mxflashattn_amd.workloads import make_paged_batch
+from oracle import reference_port
+
+TOL = {torch.float16: 2e-3, torch.bfloat16: 1.6e-2}
+FP8 = torch.float8_e4m3fn
+
+
+def test_launch_columns_and_token_shares():
+    assert native.launch_columns(64, 16, False, True) == 64
+    assert native.launch_columns(128, 16, False, False) == 48
+    assert native.launch_columns(128, 16, False, True) == 32
+    assert native.launch_columns(64, 16, True, False) == 32
+    assert native.launch_columns(128, 256, True, True) == 32
+    assert native.launch_columns(256, 16, False, False) == 16
+    assert native.launch_columns(128, 8, False, False) == 16   # per-lane page ids
+    # Full launches of 16 columns; about equal shares of several groups.
+    assert native.tokens_per_launch(5, 4, 16) == 4
+    assert native.tokens_per_launch(16, 4, 48) == 8            # 64 columns: 2 x 32
+    assert native.tokens_per_launch(12, 4, 48) == 12
+    assert native.tokens_per_launch(64, 1, 48) == 32
+    assert native.tokens_per_launch(4, 16, 48) == 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("ql,gq", [(17, 1), (31, 1), (16, 2), (11, 3), (33, 1), (47, 1), (12, 4),
+                                   (49, 1), (9, 7), (64, 1), (4, 16)])
+@pytest.mark.parametrize("mode", ["plain", "options", "fp8"])
+def test_column_group_edges(device, head_dim, ql, gq, mode):
+    dtype = torch.float16 if (ql + gq) % 2 else torch.bfloat16
+    # Shorter than the query, on and beside a tile's edge, several ranges long.
+    lens = torch.tensor([1, ql, 16, 0, 511, 1300])
+    b = make_paged_batch(6, 2 * gq, 2, head_dim, dtype, lens, seed=200 + ql, q_len=ql)
+    k, v = b.k_cache, b.v_cache
+    if mode == "fp8":
+        k, v = k.to(FP8), v.to(FP8)
+    opts = {}
+    if mode == "options":
+        opts = dict(window_left=70, softcap=20.0, sinks=torch.linspace(-2, 3, 2 * gq),
+                    alibi_slopes=torch.logspace(-1, -6, 2 * gq, base=2.0))
+    live = lens > 0
+    ref = reference_port.attention_kvcache(
+        b.q[live].float(), k.float(), v.float(), cache_seqlens=b.cache_seqlens[live],
+        block_table=b.block_table[live], softmax_scale=b.scale, causal=True, **opts)
+    expected = torch.zeros(b.q.shape)
+    expected[live] = ref.float()
+    kw = {n: t.to(device) if isinstance(t, torch.Tensor) else t for n, t in opts.items()}
+    g = b.to(device)
+    for ns in (None, 1, 7, 300):
+        out = native.paged_decode_split(g.q, k.to(device), v.to(device), g.block_table,
+                                        g.cache_seqlens, g.scale, causal=True, num_splits=ns, **kw)
+        err = (out.float().cpu() - expected).abs().max().item()
+        assert err <= TOL[dtype], (ns, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [64, 65, 300])
+def test_column_groups_on_both_tile_scans(device, batch):
+    # Up to 64 sequences the waves scan the tiles themselves, past that through LDS.
+    g = torch.Generator().manual_seed(batch)
+    lens = torch.randint(6, 80, (batch,), generator=g)
+    b = make_paged_batch(batch, 20, 5, 128, torch.bfloat16, lens, seed=batch, q_len=6,
+                         page_size=32)
+    ref = reference_port.attention_kvcache(
+        b.q.float(), b.k_cache.float(), b.v_cache.float(), cache_seqlens=b.cache_seqlens,
+        block_table=b.block_table, softmax_scale=b.scale, causal=True).float()
+    d = b.to(device)
+    out = native.paged_decode_split(d.q, d.k_cache, d.v_cache, d.block_table, d.cache_seqlens,
+                                    d.scale, causal=True, num_splits=100)
+    assert (out.float().cpu() - ref).abs().max().item() <= TOL[torch.bfloat16]
