@@ -150,7 +150,7 @@ def flash_attn_varlen_func(
             "return_attn_probs": return_attn_probs,
         },
         decode_route=decode.route_varlen(q, k, v, cu_seqlens_k, q_offsets, k_offsets,
-                                         max_seqlen_k, scale, causal),
+                                         max_seqlen_k, scale, causal, cu_seqlens_q),
     )
 
 

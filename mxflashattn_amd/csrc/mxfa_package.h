@@ -31,6 +31,30 @@ int mxfa_package_decode_tokens_launch(
     int block_table_width, int num_pages, int dtype, int kv_dtype, const float *k_scale,
     const float *v_scale, int num_splits, void *stream);
 
+// Decode over keys that lie in consecutive rows, read in place (16-bit caches):
+// k and v rows of kv head h at first_stride * first(b) + token_stride * i +
+// head_stride * h elements for token i of sequence b.
+//   dense (cu_seqlens_k null): first(b) = b (first_stride: the batch stride;
+//     num_firsts: the batch dimension of k), max_len keys each, or
+//     seqlens[b] + seqlen_add (at most max_len);
+//   packed (cu_seqlens_q, cu_seqlens_k of num_seqs + 1 offsets, int32 or
+//     int64): the query rows are the sequences with cu_q[i + 1] > cu_q[i], in
+//     order; first_stride = token_stride, num_firsts the total of key rows.
+// Any number of causal query tokens, as many per launch as the kernel takes.
+// One small launch writes first rows and lengths to the workspace's tail;
+// workspace from mxfa_package_contiguous_workspace_size.
+int mxfa_package_contiguous_workspace_size(int batch, int q_heads, int kv_heads, int q_len,
+                                           int head_dim, int num_splits, size_t *bytes);
+int mxfa_package_contiguous_decode_launch(
+    const void *q, int64_t q_stride_b, int64_t q_stride_t, int64_t q_stride_h, int q_len,
+    int causal, const void *k, const void *v, int64_t first_stride, int64_t token_stride,
+    int64_t head_stride, int64_t num_firsts, int max_len, const void *cu_seqlens_q,
+    int cu_q_is_int64, const void *cu_seqlens_k, int cu_k_is_int64, int num_seqs,
+    const int32_t *seqlens, int seqlen_add, void *out, int64_t out_stride_b,
+    int64_t out_stride_t, int64_t out_stride_h, void *workspace, size_t workspace_bytes,
+    float scale, int batch, int q_heads, int kv_heads, int head_dim, int dtype, int num_splits,
+    void *stream);
+
 #ifdef __cplusplus
 }
 #endif

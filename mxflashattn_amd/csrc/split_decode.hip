@@ -138,6 +138,8 @@ struct SplitArgs {
   const float *alibi;  // per query head ALiBi slopes, nullptr: none
   int min_seqlen_add;  // 0, or -2^30 where lengths below zero count as 0
   int max_cols;        // columns (query tokens x heads per kv head) the entry point takes
+  bool contiguous;     // a sequence's keys are consecutive rows: one page per sequence (ps 1,
+                       // btw = the longest sequence, bt = its first row or page, bt_stride 1)
 };
 
 struct WsLayout {
@@ -262,7 +264,7 @@ static DecodeParams make_params(const SplitArgs &a, const Grid &g) {
   p.alibi = a.alibi;
   p.heads_per_wg = g.heads_per_wg;
   p.subs = g.subs;
-  p.ps_log2 = ilog2_exact(a.ps);
+  p.ps_log2 = a.contiguous ? kContiguousLog2 : ilog2_exact(a.ps);
   p.max_len = a.btw * a.ps;
   p.num_pages = a.num_pages;
   p.num_ranges = a.num_splits;
@@ -411,6 +413,7 @@ static SplitArgs split_args(const void *q, int64_t q_stride_b, int64_t q_stride_
   a.alibi = nullptr;
   a.min_seqlen_add = 0;
   a.max_cols = kMaxCols;
+  a.contiguous = false;
   return a;
 }
 
@@ -520,6 +523,75 @@ static int run_tokens(SplitArgs a, int64_t q_stride_t, int q_len, int causal, in
     a.max_cols = launch_columns(a.hd, a.ps, a.fp8,
                                 window_left >= 0 || softcap > 0.f || sinks || alibi_slopes);
   return run_split(a, true, st);
+}
+
+// First rows and lengths of sequences whose keys are consecutive rows, for the
+// decode kernels' block table and lengths. One workgroup: a few hundred to
+// 16,000 entries, latency-bound (about 2 us, where building the same as a
+// table of one-token pages took four or five elementwise launches and 4 bytes
+// a key). Measured on MI355X against that table and its per-lane page ids (us
+// a call through the API, same outputs bit for bit): 32 packed sequences of
+// 1k-8k keys, 32q/8kv HD 128, 188.0 -> 157.8, the split kernel itself 122.5 ->
+// 108.5; 16 dense sequences of 4095 keys, 16q/8kv, 60.1 -> 46.5 (kernel 47.0 ->
+// 41.4); of 4096 keys (pages of 256 before) 52.0 -> 45.1.
+// Dense (cu_k null): sequence b is page b, max_len keys. Packed: sequence i has
+// keys [cu_k[i], cu_k[i+1]) and, if cu_q[i+1] > cu_q[i], query row cu_q[i];
+// sequences without a row are left out. Rows no sequence names get length 0,
+// and start and length are held to the total_rows rows that exist, so offsets
+// that do not describe the keys give wrong numbers, never a read outside them.
+constexpr int kRowsThreads = 1024;
+struct RowsParams {
+  const void *cu_q;
+  const void *cu_k;
+  int q64, k64;  // int64 offsets (else int32)
+  int num_seqs;
+  int64_t total_rows;
+  int max_len;
+  int batch;
+  int32_t *first;
+  int32_t *len;
+};
+
+__global__ __launch_bounds__(kRowsThreads) void contiguous_rows_kernel(RowsParams p) {
+  const auto at = [](const void *cu, int wide, int i) -> int64_t {
+    return wide ? static_cast<const int64_t *>(cu)[i] : static_cast<const int32_t *>(cu)[i];
+  };
+  for (int r = threadIdx.x; r < p.batch; r += kRowsThreads) {
+    p.first[r] = p.cu_k ? 0 : r;
+    p.len[r] = p.cu_k ? 0 : p.max_len;
+  }
+  if (!p.cu_k) return;
+  __syncthreads();
+  for (int i = threadIdx.x; i < p.num_seqs; i += kRowsThreads) {
+    const int64_t r = at(p.cu_q, p.q64, i), r1 = at(p.cu_q, p.q64, i + 1);
+    if (r1 <= r || r < 0 || r >= p.batch) continue;
+    const int64_t k0 = at(p.cu_k, p.k64, i), k1 = at(p.cu_k, p.k64, i + 1);
+    const int64_t first = k0 < 0 ? 0 : k0 > p.total_rows ? p.total_rows : k0;
+    int64_t n = k1 - first;
+    n = n > p.total_rows - first ? p.total_rows - first : n;
+    n = n > p.max_len ? p.max_len : n;
+    p.first[r] = (int32_t)first;
+    p.len[r] = n > 0 ? (int32_t)n : 0;
+  }
+}
+
+// Workspace of a contiguous call: the split workspace of `rows` = q heads x
+// query tokens of one launch, then first rows and lengths.
+static size_t contiguous_ws(int batch, int rows, int hd, int ns, size_t *tail) {
+  const size_t split = ns > 0 ? ws_layout(batch, rows, hd, ns).bytes : 0;
+  *tail = (split + 15) & ~(size_t)15;
+  return *tail + (size_t)batch * 2 * sizeof(int32_t);
+}
+
+// Query tokens of one launch of a contiguous call: all of them, or for a
+// causal query of more columns as many as fit (about equal shares where a
+// launch takes several column groups).
+static int contiguous_tokens(int ql, int gq, int hd, int ns) {
+  const int cols = ns > 0 ? launch_columns(hd, kTile, false, false) : kMaxCols;
+  const int most = cols / gq;
+  if (ql <= most || cols == kMaxCols) return ql < most ? ql : most;
+  const int launches = (ql + most - 1) / most;
+  return (ql + launches - 1) / launches;
 }
 
 }  // namespace mxfa
@@ -714,6 +786,74 @@ int mxfa_package_decode_tokens_launch(
   return run_tokens(split_args(MXFA_SPLIT_ARGS), q_stride_t, q_len, causal, window_left, sinks,
                     softcap, alibi_slopes, out_stride_t, kv_dtype, k_scale, v_scale, true,
                     (hipStream_t)stream);
+}
+
+int mxfa_package_contiguous_workspace_size(int batch, int q_heads, int kv_heads, int q_len,
+                                           int head_dim, int num_splits, size_t *bytes) {
+  if (!bytes || batch <= 0 || q_heads <= 0 || kv_heads <= 0 || q_len <= 0 || head_dim <= 0 ||
+      q_heads % kv_heads || q_heads / kv_heads > kMaxCols ||
+      (num_splits <= 0 && num_splits != MXFA_SPLITS_PER_SEQUENCE))
+    return MXFA_EINVAL;
+  const int tokens = contiguous_tokens(q_len, q_heads / kv_heads, head_dim, num_splits);
+  size_t tail;
+  *bytes = contiguous_ws(batch, q_heads * tokens, head_dim, num_splits, &tail);
+  return MXFA_OK;
+}
+
+int mxfa_package_contiguous_decode_launch(
+    const void *q, int64_t q_stride_b, int64_t q_stride_t, int64_t q_stride_h, int q_len,
+    int causal, const void *k, const void *v, int64_t first_stride, int64_t token_stride,
+    int64_t head_stride, int64_t num_firsts, int max_len, const void *cu_seqlens_q,
+    int cu_q_is_int64, const void *cu_seqlens_k, int cu_k_is_int64, int num_seqs,
+    const int32_t *seqlens, int seqlen_add, void *out, int64_t out_stride_b,
+    int64_t out_stride_t, int64_t out_stride_h, void *workspace, size_t workspace_bytes,
+    float scale, int batch, int q_heads, int kv_heads, int head_dim, int dtype, int num_splits,
+    void *stream) {
+  size_t need = 0;
+  int rc = mxfa_package_contiguous_workspace_size(batch, q_heads, kv_heads, q_len, head_dim,
+                                                  num_splits, &need);
+  if (rc != MXFA_OK) return rc;
+  if (!workspace || !aligned16(workspace) || workspace_bytes < need) return MXFA_EWORKSPACE;
+  if (num_firsts <= 0 || num_firsts > INT32_MAX || max_len <= 0) return MXFA_EINVAL;
+  if (cu_seqlens_k ? (!cu_seqlens_q || num_seqs < batch || seqlens) : num_firsts < batch)
+    return MXFA_EINVAL;
+  const int tokens = contiguous_tokens(q_len, q_heads / kv_heads, head_dim, num_splits);
+  if (tokens < q_len && !causal) return MXFA_EUNSUPPORTED;
+  size_t tail = 0;
+  contiguous_ws(batch, q_heads * tokens, head_dim, num_splits, &tail);
+  int32_t *first = (int32_t *)((char *)workspace + tail);
+  SplitArgs a = split_args(q, q_stride_b, q_stride_h, k, v, first_stride, token_stride,
+                           head_stride, first, 1, seqlens ? seqlens : first + batch, seqlen_add,
+                           out, out_stride_b, out_stride_h, workspace, tail, scale, batch,
+                           q_heads, kv_heads, head_dim, 1, max_len, (int)num_firsts, dtype,
+                           num_splits);
+  a.contiguous = true;
+  a.q_st = q_stride_t;
+  a.o_st = out_stride_t;
+  a.causal = causal;
+  a.min_seqlen_add = -(1 << 30);
+  if (num_splits > 0) a.max_cols = launch_columns(head_dim, kTile, false, false);
+  const hipStream_t st = (hipStream_t)stream;
+  // A causal query of several launches: tokens [t, t + n) run as the last n
+  // tokens of sequences shortened by the tokens after them.
+  for (int t = 0; t < q_len; t += tokens) {
+    const int n = q_len - t < tokens ? q_len - t : tokens;
+    a.q = (const char *)q + (int64_t)t * q_stride_t * 2;
+    a.out = (char *)out + (int64_t)t * out_stride_t * 2;
+    a.ql = n;
+    a.seqlen_add = seqlen_add - (q_len - t - n);
+    if (t == 0) {
+      rc = check_split_args(a);
+      if (rc != MXFA_OK) return rc;
+      RowsParams r{cu_seqlens_q, cu_seqlens_k, cu_q_is_int64, cu_k_is_int64, num_seqs,
+                   num_firsts,   max_len,      batch,         first,         first + batch};
+      hipLaunchKernelGGL(contiguous_rows_kernel, dim3(1), dim3(kRowsThreads), 0, st, r);
+      if (hipGetLastError() != hipSuccess) return MXFA_ELAUNCH;
+    }
+    rc = run_split(a, true, st);
+    if (rc != MXFA_OK) return rc;
+  }
+  return MXFA_OK;
 }
 
 int mxfa_package_launch_columns(int head_dim, int page_size, int fp8, int extras) {

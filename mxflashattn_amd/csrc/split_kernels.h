@@ -88,6 +88,10 @@ constexpr float kRescaleLog2 = 8.0f;
 // LDS: 16000 sequences keep a workgroup within 64 KB.
 constexpr int kMaxBatch = 16000;
 constexpr int kMaxCols = 16;      // query tokens x heads per kv head: the 16 MFMA columns of a group
+// log2 of the page size that stands for keys in consecutive rows: no sequence
+// is longer (lengths are at most 2^30), so the block-table index is always 0
+// and a tile's offset in its page is its offset in the sequence.
+constexpr int kContiguousLog2 = 30;
 constexpr int kOffOut = 0x40000000;          // a lane offset no descriptor covers
 
 // Tile flags.
@@ -1857,7 +1861,9 @@ static int launch_partial_hr(const DecodeParams &p, const Grid &g, hipStream_t s
   switch (head_rows(cols)) {
     case 1:
       if constexpr (!kF8 && HD >= 128) {
-        if (p.ps_log2 >= 4) {
+        // Keys in consecutive rows take QK on the matrix cores: the same bits
+        // as the same keys read as one-token pages (about 0.5 % of a call).
+        if (p.ps_log2 >= 4 && p.ps_log2 != kContiguousLog2) {
           switch (valu_qk_columns(cols, HD)) {
             case 1: return launch_partial_t<HD, 1, T, kF8, kWaveScan, 1>(p, g, st);
             case 2: return launch_partial_t<HD, 1, T, kF8, kWaveScan, 2>(p, g, st);

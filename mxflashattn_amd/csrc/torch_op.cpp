@@ -33,6 +33,7 @@
 #include <vector>
 
 #include "mxfa_mi355x.h"
+#include "mxfa_package.h"
 
 namespace {
 
@@ -207,6 +208,124 @@ py::object decode(const at::Tensor &q, const at::Tensor &k_cache, const at::Tens
   return py::cast(out);
 }
 
+// contiguous_decode(q, k, v, scale, causal, max_len, cu_seqlens_q,
+// cu_seqlens_k, seqlens, out): decode over keys in consecutive rows, read in
+// place (mxfa_package_contiguous_decode_launch).
+//   dense: q [B, QL, HQ, HD], k and v [B, S, HKV, HD], every sequence max_len =
+//     S keys, or seqlens (int32 [B]) of them;
+//   packed (cu_seqlens_q and cu_seqlens_k given): q [B, HQ, HD], the B rows of
+//     the sequences that have one, k and v [T, HKV, HD].
+// Returns the output, or None (nothing launched) for calls whose tensors the
+// kernels do not read in place.
+py::object contiguous_decode(const at::Tensor &q, const at::Tensor &k, const at::Tensor &v,
+                             double scale, bool causal, int64_t max_len,
+                             const c10::optional<at::Tensor> &cu_q_arg,
+                             const c10::optional<at::Tensor> &cu_k_arg,
+                             const c10::optional<at::Tensor> &seqlens_arg,
+                             const c10::optional<at::Tensor> &out_arg) {
+  const bool packed = cu_q_arg.has_value();
+  const int64_t rank = packed ? 3 : 4;
+  const at::ScalarType dt = q.scalar_type();
+  if ((dt != at::kHalf && dt != at::kBFloat16) || k.scalar_type() != dt || v.scalar_type() != dt)
+    return py::none();
+  if (!q.is_cuda() || q.dim() != rank || k.dim() != rank || !v.sizes().equals(k.sizes()) ||
+      !v.strides().equals(k.strides()) || k.stride(-1) != 1 || q.stride(-1) != 1)
+    return py::none();
+  const at::Device device = q.device();
+  if (k.device() != device || v.device() != device || device.index() != c10::hip::current_device())
+    return py::none();
+  const int64_t batch = q.size(0), ql = packed ? 1 : q.size(1);
+  const int64_t hq = q.size(-2), hkv = k.size(-2), hd = q.size(-1);
+  const int64_t firsts = k.size(0);
+  if (batch < 1 || ql < 1 || hkv < 1 || hq % hkv || hq / hkv > 16 || k.size(-1) != hd ||
+      max_len < 1 || max_len > 1 << 30 || firsts > std::numeric_limits<int>::max())
+    return py::none();
+  const auto vector_on_device = [&](const at::Tensor &t) {
+    return t.device() == device && t.dim() == 1 && t.is_contiguous();
+  };
+  const void *cu_q = nullptr, *cu_k = nullptr;
+  const int32_t *seqlens = nullptr;
+  bool cu_q64 = false, cu_k64 = false;
+  int64_t num_seqs = batch;
+  if (packed) {
+    if (!cu_k_arg.has_value()) return py::none();
+    const at::Tensor &tq = *cu_q_arg, &tk = *cu_k_arg;
+    for (const at::Tensor *t : {&tq, &tk})
+      if (!vector_on_device(*t) || (t->scalar_type() != at::kInt && t->scalar_type() != at::kLong))
+        return py::none();
+    num_seqs = tq.numel() - 1;
+    if (tk.numel() != tq.numel() || num_seqs < batch) return py::none();
+    cu_q = tq.data_ptr();
+    cu_k = tk.data_ptr();
+    cu_q64 = tq.scalar_type() == at::kLong;
+    cu_k64 = tk.scalar_type() == at::kLong;
+  } else {
+    if (firsts < batch || max_len > k.size(1)) return py::none();
+    if (seqlens_arg.has_value()) {
+      const at::Tensor &t = *seqlens_arg;
+      if (!vector_on_device(t) || t.scalar_type() != at::kInt || t.numel() != batch)
+        return py::none();
+      seqlens = t.data_ptr<int32_t>();
+    }
+  }
+  // q's and the output's strides (batch, token, head); a token stride of one
+  // token is never used, so it need not suit the kernel.
+  const auto strides = [&](const at::Tensor &t, int64_t (&s)[3]) {
+    s[0] = t.stride(0);
+    s[1] = ql > 1 ? t.stride(1) : 0;
+    s[2] = t.stride(-2);
+  };
+  int64_t qs[3], os[3];
+  strides(q, qs);
+  if (!aligned(q.data_ptr(), 16) || ((qs[0] | qs[1] | qs[2]) & 7) || (hq > 1 && qs[2] < hd))
+    return py::none();
+  at::Tensor out;
+  if (out_arg.has_value()) {
+    out = *out_arg;
+    if (out.scalar_type() != dt || out.device() != device || !out.sizes().equals(q.sizes()) ||
+        out.stride(-1) != 1)
+      return py::none();
+    strides(out, os);
+    if (!aligned(out.data_ptr(), 8) || ((os[0] | os[1] | os[2]) & 3)) return py::none();
+  } else {
+    out = at::empty(q.sizes(), q.options());
+    strides(out, os);
+  }
+  // The heuristic as for pages of 16 tokens, asked for the columns of one
+  // launch; past 16 columns it is asked again unless it picked the
+  // per-sequence kernel.
+  const int cus = num_cus(device.index()), width = (int)((max_len + 15) / 16);
+  const int64_t gq = hq / hkv;
+  const int64_t first_ask = std::min<int64_t>(ql, std::max<int64_t>(1, 16 / gq));
+  int ns = 0;
+  if (mxfa_split_heuristic((int)batch, (int)(hq * first_ask), (int)hkv, (int)hd, 16, width, cus,
+                           &ns) != MXFA_OK)
+    return py::none();
+  if (first_ask < ql && ns != MXFA_SPLITS_PER_SEQUENCE &&
+      mxfa_split_heuristic((int)batch, (int)(hkv * 17), (int)hkv, (int)hd, 16, width, cus, &ns) !=
+          MXFA_OK)
+    return py::none();
+  size_t ws_bytes = 0;
+  if (mxfa_package_contiguous_workspace_size((int)batch, (int)hq, (int)hkv, (int)ql, (int)hd, ns,
+                                             &ws_bytes) != MXFA_OK)
+    return py::none();
+  void *stream = (void *)c10::hip::getCurrentHIPStream(device.index()).stream();
+  at::Tensor ws = workspace(device, stream, ws_bytes);
+  poison(stream, out, &ws);
+  const int64_t token_stride = k.stride(packed ? 0 : 1);
+  const int rc = mxfa_package_contiguous_decode_launch(
+      q.data_ptr(), qs[0], qs[1], qs[2], (int)ql, causal, k.data_ptr(), v.data_ptr(), k.stride(0),
+      token_stride, k.stride(-2), firsts, (int)max_len, cu_q, cu_q64, cu_k, cu_k64, (int)num_seqs,
+      seqlens, 0, out.data_ptr(), os[0], os[1], os[2], ws.data_ptr(), ws_bytes, (float)scale,
+      (int)batch, (int)hq, (int)hkv, (int)hd, dt == at::kBFloat16 ? MXFA_DTYPE_BF16 : MXFA_DTYPE_F16,
+      ns, stream);
+  if (rc == MXFA_EUNSUPPORTED || rc == MXFA_EINVAL) return py::none();  // nothing launched
+  if (rc != MXFA_OK)
+    throw std::runtime_error(std::string("contiguous decode failed (") + std::to_string(rc) +
+                             "): " + mxfa_strerror(rc));
+  return py::cast(out);
+}
+
 // reshape_and_cache(key, value, key_cache, value_cache, slot_mapping): the
 // vLLM-form append of 16-bit caches (mxfa_reshape_and_cache_launch) for the
 // common call: key/value [T, HKV, HD] sharing strides with a contiguous last
@@ -259,6 +378,10 @@ PYBIND11_MODULE(_mxfa_torch, m) {
         py::arg("block_table"), py::arg("cache_seqlens"), py::arg("scale"),
         py::arg("out") = py::none(), py::arg("num_splits") = py::none(),
         py::arg("seqlen_add") = 0);
+  m.def("contiguous_decode", &contiguous_decode, py::arg("q"), py::arg("k"), py::arg("v"),
+        py::arg("scale"), py::arg("causal"), py::arg("max_len"),
+        py::arg("cu_seqlens_q") = py::none(), py::arg("cu_seqlens_k") = py::none(),
+        py::arg("seqlens") = py::none(), py::arg("out") = py::none());
   m.def("reshape_and_cache", &reshape_and_cache, py::arg("key"), py::arg("value"),
         py::arg("key_cache"), py::arg("value_cache"), py::arg("slot_mapping"));
   m.def("abi_version", &mxfa_abi_version);

@@ -15,12 +15,14 @@ not synchronise the stream.
   flash_attn_func          q_len QL with QL * GQ <= 16: k/v [B, S, HKV, D] is a
                            dense cache of S tokens per sequence.
   flash_attn_varlen_func   every sequence has at most one query token: packed
-                           k/v are a cache of one-token pages whose block table
-                           row b is cu_seqlens_k[b] + arange(max_seqlen_k).
+                           k/v, sequence b's keys at rows cu_seqlens_k[b] on.
 
-A dense cache [B, S, HKV, D] is viewed as pages of P tokens, P the largest
-power of two dividing S (capped at 256), with block table row b =
-b * S/P + arange(S/P): the same bytes, no copy.
+Dense and packed keys lie in consecutive rows, which the operator's
+contiguous_decode reads in place. What it does not take (an append to a dense
+cache, tensors it cannot read in place) runs over pages of the same bytes: a
+dense cache [B, S, HKV, D] as pages of P tokens, P the largest power of two
+dividing S (capped at 256), with block table row b = b * S/P + arange(S/P);
+packed keys as one-token pages with row b = cu_seqlens_k[b] + arange(longest).
 """
 
 from __future__ import annotations
@@ -80,6 +82,17 @@ def _dense_table(batch: int, pages_per_seq: int, device: torch.device) -> torch.
     return base + torch.arange(pages_per_seq, device=device, dtype=torch.int32).unsqueeze(0)
 
 
+def _contiguous(q, k, v, scale, causal, max_len, cu_seqlens_q=None, cu_seqlens_k=None,
+                seqlens=None, out=None) -> torch.Tensor | None:
+    """The operator's decode over keys in consecutive rows, or None (nothing
+    launched) when it does not take the call."""
+    op = native.torch_op() if native.USE_TORCH_OP else None
+    if op is None:
+        return None
+    return op.contiguous_decode(q, k, v, scale, bool(causal), max_len, cu_seqlens_q,
+                                cu_seqlens_k, seqlens, out)
+
+
 def route_kvcache(q, k_cache, v_cache, k, v, cache_seqlens, block_table, scale,
                   causal, out: torch.Tensor | None = None) -> DecodeRoute:
     """``out`` (q's shape and dtype, last dim contiguous) receives the result
@@ -108,6 +121,11 @@ def route_kvcache(q, k_cache, v_cache, k, v, cache_seqlens, block_table, scale,
         k, v = k.contiguous(), v.contiguous()
 
     def run() -> torch.Tensor:
+        if block_table is None and k is None:
+            result = _contiguous(q, k_cache, v_cache, scale, causal, k_cache.shape[1],
+                                 seqlens=cache_seqlens, out=out)
+            if result is not None:
+                return result
         if block_table is None:
             table = _dense_table(q.shape[0], kc.shape[0] // q.shape[0], q.device)
         else:
@@ -137,6 +155,9 @@ def route_dense(q, k, v, scale, causal) -> DecodeRoute:
         return DecodeRoute(reason)
 
     def run() -> torch.Tensor:
+        result = _contiguous(q, k, v, scale, causal, k.shape[1])
+        if result is not None:
+            return result
         batch = q.shape[0]
         table = _dense_table(batch, kc.shape[0] // batch, q.device)
         lengths = torch.full((batch,), k.shape[1], dtype=torch.int32, device=q.device)
@@ -146,11 +167,10 @@ def route_dense(q, k, v, scale, causal) -> DecodeRoute:
 
 
 def route_varlen(q, k, v, cu_seqlens_k: torch.Tensor, q_offsets: list[int], k_offsets: list[int],
-                 max_seqlen_k: int, scale, causal) -> DecodeRoute:
+                 max_seqlen_k: int, scale, causal,
+                 cu_seqlens_q: torch.Tensor | None = None) -> DecodeRoute:
     """Packed decode: sequence b's keys are rows [cu_k[b], cu_k[b+1]) of k/v,
-    read in place as one-token pages. The block table and lengths are built
-    on the device from ``cu_seqlens_k`` (no host-to-device copy) when every
-    sequence has its query row, the usual decode batch."""
+    read in place (first rows and lengths come from the offsets on the device)."""
     reason = _common_reason(q, k.shape[1], q.shape[-1])
     if reason is not None:
         return DecodeRoute(reason)
@@ -173,6 +193,10 @@ def route_varlen(q, k, v, cu_seqlens_k: torch.Tensor, q_offsets: list[int], k_of
         return DecodeRoute(reason)
 
     def run() -> torch.Tensor:
+        if cu_seqlens_q is not None:
+            result = _contiguous(q, k, v, scale, False, width, cu_seqlens_q, cu_seqlens_k)
+            if result is not None:
+                return result
         device = q.device
         cu = cu_seqlens_k.to(torch.int32)
         starts, lengths = cu[:-1], cu[1:] - cu[:-1]

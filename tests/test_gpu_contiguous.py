@@ -1,0 +1,120 @@
+"""Keys in consecutive rows read in place (dense caches and packed sequences):
+the operator's contiguous_decode against the reference port, and the paged
+route of the same call, over the layouts both take."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import mxflashattn_amd as mx
+from mxflashattn_amd import native
+from oracle import reference_port
+
+TOL = {torch.float16: 2e-3, torch.bfloat16: 1.6e-2}
+
+pytestmark = pytest.mark.gpu
+
+
+def randn(*shape, dtype, seed):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(dtype)
+
+
+def close(got, expected, dtype):
+    err = (got.float().cpu() - expected.float()).abs().max().item()
+    assert err <= TOL[dtype], err
+
+
+def both_routes(monkeypatch, call):
+    """The call through the operator and through the paged route."""
+    out = call()
+    assert mx.get_last_dispatch_info().backend == mx.BACKEND_MI355X
+    monkeypatch.setattr(native, "USE_TORCH_OP", False)
+    paged = call()
+    monkeypatch.undo()
+    return out, paged
+
+
+@pytest.mark.parametrize("hd,gq,dtype", [(64, 1, torch.float16), (64, 8, torch.bfloat16),
+                                         (128, 2, torch.float16), (128, 4, torch.bfloat16),
+                                         (128, 16, torch.bfloat16)])
+@pytest.mark.parametrize("wide", [False, True], ids=["int32", "int64"])
+def test_packed_rows(device, monkeypatch, hd, gq, dtype, wide):
+    hkv = 3
+    lens = [1, 15, 16, 17, 700, 33, 1900, 5]
+    rows = [1, 1, 0, 1, 1, 0, 1, 1]  # sequences 2 and 5 have no query row
+    kv = randn(sum(lens), 2, hkv, hd, dtype=dtype, seed=hd + gq)  # K and V rows interleaved
+    q = randn(sum(rows), hkv * gq + 1, hd, dtype=dtype, seed=gq)[:, 1:]
+    cu_q = torch.tensor([0, *torch.tensor(rows).cumsum(0).tolist()])
+    cu_k = torch.tensor([0, *torch.tensor(lens).cumsum(0).tolist()])
+    ref = reference_port.attention_varlen(q.float(), kv[:, 0].float(), kv[:, 1].float(),
+                                          cu_q.tolist(), cu_k.tolist(), softmax_scale=hd ** -0.5)
+    dt = torch.int64 if wide else torch.int32
+    d = kv.to(device)
+    qd = torch.empty(sum(rows), hkv * gq + 1, hd, dtype=dtype, device=device)
+    qd[:, 1:] = q.to(device)
+    out, paged = both_routes(monkeypatch, lambda: mx.flash_attn_varlen_func(
+        qd[:, 1:], d[:, 0], d[:, 1], cu_q.to(device, dt), cu_k.to(device, dt), 1, max(lens)))
+    close(out, ref, dtype)
+    assert torch.equal(out, paged)  # the same tiles, ranges and arithmetic
+
+
+def test_short_packed_sequences_take_the_per_sequence_kernel(device):
+    lens = [1, 16, 200, 255, 31]
+    k, v = (randn(sum(lens), 2, 64, dtype=torch.float16, seed=s) for s in (1, 2))
+    q = randn(5, 8, 64, dtype=torch.float16, seed=3)
+    cu_q, cu_k = torch.arange(6), torch.tensor([0, *torch.tensor(lens).cumsum(0).tolist()])
+    ref = reference_port.attention_varlen(q.float(), k.float(), v.float(), cu_q.tolist(),
+                                          cu_k.tolist(), softmax_scale=0.125)
+    out = mx.flash_attn_varlen_func(q.to(device), k.to(device), v.to(device), cu_q.to(device),
+                                    cu_k.to(device), 1, 255)
+    close(out, ref, torch.float16)
+
+
+@pytest.mark.parametrize("seq", [1, 15, 47, 96, 1025, 2048])
+@pytest.mark.parametrize("hd,gq,ql,dtype", [(64, 2, 1, torch.float16), (128, 4, 1, torch.bfloat16),
+                                            (128, 1, 3, torch.bfloat16), (64, 4, 9, torch.float16),
+                                            (128, 4, 16, torch.bfloat16)])
+def test_dense_rows(device, monkeypatch, seq, hd, gq, ql, dtype):
+    if ql > seq:
+        pytest.skip("fewer keys than query tokens")
+    kv = randn(3, seq, 2, 2, hd, dtype=dtype, seed=seq)  # token rows of K and V interleaved
+    q = randn(3, ql, 2 * gq, hd, dtype=dtype, seed=ql)
+    ref = reference_port.attention_batched(q.float(), kv[:, :, 0].float(), kv[:, :, 1].float(),
+                                           softmax_scale=hd ** -0.5, causal=True)
+    d = kv.to(device)
+    out, paged = both_routes(monkeypatch, lambda: mx.flash_attn_func(
+        q.to(device), d[:, :, 0], d[:, :, 1], causal=True))
+    close(out, ref, dtype)
+    close(paged, ref, dtype)
+    # The cache entry point: lengths of its own, some empty, into a given output.
+    lens = torch.tensor([seq, (seq + 1) // 2, 0], dtype=torch.int32)
+    buf = torch.full((3, ql, 2 * gq + 3, hd), 7.0, device=device, dtype=dtype)
+    got = mx.flash_attn_with_kvcache(q.to(device), d[:, :, 0], d[:, :, 1],
+                                     cache_seqlens=lens.to(device), causal=True,
+                                     out=buf[:, :, 1:-2])
+    assert got.data_ptr() == buf[:, :, 1:-2].data_ptr()
+    for b in range(3):
+        n = int(lens[b])
+        want = torch.zeros(ql, 2 * gq, hd) if n == 0 else reference_port.attention_single(
+            q[b].float(), kv[b, :n, 0].float(), kv[b, :n, 1].float(), softmax_scale=hd ** -0.5,
+            causal=True)
+        close(got[b], want, dtype)
+    assert (buf[:, :, :1] == 7).all() and (buf[:, :, -2:] == 7).all()
+
+
+def test_offsets_that_name_no_keys_read_nothing_outside(device):
+    # The operator itself, past the API's checks: offsets that run backwards,
+    # start before the keys or end after them are held to the rows that exist.
+    op = native.torch_op()
+    k, v = (randn(100, 2, 64, dtype=torch.float16, seed=s).to(device) for s in (5, 6))
+    q = randn(4, 4, 64, dtype=torch.float16, seed=7).to(device)
+    cu_q = torch.arange(5, dtype=torch.int32, device=device)
+    cu_k = torch.tensor([-50, 90, 5000, 40, 100], dtype=torch.int32, device=device)
+    out = op.contiguous_decode(q, k, v, 0.125, False, 128, cu_q, cu_k)
+    ref = [(0, 90), (90, 100), (0, 0), (40, 100)]
+    for b, (a, e) in enumerate(ref):
+        want = torch.zeros(4, 64) if a == e else reference_port.attention_single(
+            q[b:b + 1].float().cpu(), k[a:e].float().cpu(), v[a:e].float().cpu(),
+            softmax_scale=0.125)[0]
+        close(out[b], want, torch.float16)
