@@ -119,8 +119,13 @@ def flash_attn_varlen_func(
     if cu_seqlens_q.device != q.device or cu_seqlens_k.device != q.device:
         raise ValueError("cu_seqlens_q and cu_seqlens_k must be on the same device as q")
     _options(dropout_p, window_size, softcap, alibi_slopes, deterministic, return_attn_probs)
+    scale = _resolved_scale(q.shape[-1], softmax_scale)
+    started, q_values, k_values = decode.start_varlen(
+        q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, scale
+    ) or (None, None, None)
     q_offsets = validate_cumulative_lengths(
-        cu_seqlens_q, total_tokens=q.shape[0], max_seqlen=max_seqlen_q, name="cu_seqlens_q"
+        cu_seqlens_q, total_tokens=q.shape[0], max_seqlen=max_seqlen_q, name="cu_seqlens_q",
+        values=q_values,
     )
     k_offsets = validate_cumulative_lengths(
         cu_seqlens_k,
@@ -128,10 +133,10 @@ def flash_attn_varlen_func(
         max_seqlen=max_seqlen_k,
         name="cu_seqlens_k",
         require_non_empty=True,
+        values=k_values,
     )
     if len(q_offsets) != len(k_offsets):
         raise ValueError("cu_seqlens_q and cu_seqlens_k must describe the same batch size")
-    scale = _resolved_scale(q.shape[-1], softmax_scale)
     return dispatch(
         "flash_attn_varlen_func",
         q,
@@ -150,7 +155,7 @@ def flash_attn_varlen_func(
             "return_attn_probs": return_attn_probs,
         },
         decode_route=decode.route_varlen(q, k, v, cu_seqlens_k, q_offsets, k_offsets,
-                                         max_seqlen_k, scale, causal, cu_seqlens_q),
+                                         max_seqlen_k, scale, causal, cu_seqlens_q, started),
     )
 
 

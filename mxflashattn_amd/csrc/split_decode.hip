@@ -550,6 +550,7 @@ struct RowsParams {
   int batch;
   int32_t *first;
   int32_t *len;
+  int64_t *host_offsets;  // host memory the device can write, or null
 };
 
 __global__ __launch_bounds__(kRowsThreads) void contiguous_rows_kernel(RowsParams p) {
@@ -562,6 +563,14 @@ __global__ __launch_bounds__(kRowsThreads) void contiguous_rows_kernel(RowsParam
   }
   if (!p.cu_k) return;
   __syncthreads();
+  // The caller's copy of the offsets (it checks them while the decode runs):
+  // num_seqs + 1 of cu_q, then of cu_k.
+  if (p.host_offsets) {
+    for (int i = threadIdx.x; i <= p.num_seqs; i += kRowsThreads) {
+      p.host_offsets[i] = at(p.cu_q, p.q64, i);
+      p.host_offsets[p.num_seqs + 1 + i] = at(p.cu_k, p.k64, i);
+    }
+  }
   for (int i = threadIdx.x; i < p.num_seqs; i += kRowsThreads) {
     const int64_t r = at(p.cu_q, p.q64, i), r1 = at(p.cu_q, p.q64, i + 1);
     if (r1 <= r || r < 0 || r >= p.batch) continue;
@@ -805,7 +814,7 @@ int mxfa_package_contiguous_decode_launch(
     int causal, const void *k, const void *v, int64_t first_stride, int64_t token_stride,
     int64_t head_stride, int64_t num_firsts, int max_len, const void *cu_seqlens_q,
     int cu_q_is_int64, const void *cu_seqlens_k, int cu_k_is_int64, int num_seqs,
-    const int32_t *seqlens, int seqlen_add, void *out, int64_t out_stride_b,
+    int64_t *host_offsets, void *offsets_event, const int32_t *seqlens, int seqlen_add, void *out, int64_t out_stride_b,
     int64_t out_stride_t, int64_t out_stride_h, void *workspace, size_t workspace_bytes,
     float scale, int batch, int q_heads, int kv_heads, int head_dim, int dtype, int num_splits,
     void *stream) {
@@ -846,9 +855,12 @@ int mxfa_package_contiguous_decode_launch(
       rc = check_split_args(a);
       if (rc != MXFA_OK) return rc;
       RowsParams r{cu_seqlens_q, cu_seqlens_k, cu_q_is_int64, cu_k_is_int64, num_seqs,
-                   num_firsts,   max_len,      batch,         first,         first + batch};
+                   num_firsts,   max_len,      batch,         first,         first + batch,
+                   host_offsets};
       hipLaunchKernelGGL(contiguous_rows_kernel, dim3(1), dim3(kRowsThreads), 0, st, r);
       if (hipGetLastError() != hipSuccess) return MXFA_ELAUNCH;
+      if (offsets_event && hipEventRecord((hipEvent_t)offsets_event, st) != hipSuccess)
+        return MXFA_ELAUNCH;
     }
     rc = run_split(a, true, st);
     if (rc != MXFA_OK) return rc;

@@ -166,11 +166,32 @@ def route_dense(q, k, v, scale, causal) -> DecodeRoute:
     return DecodeRoute(None, run)
 
 
+def start_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, scale):
+    """Launch a packed decode before its offsets are known on the host.
+
+    With max_seqlen_q = 1 the call is a decode or an error, so the kernels (which
+    hold every row they read to the rows that exist, whatever the offsets) go
+    out first, and the caller checks the offsets while they run: reading them
+    first left the GPU idle for the check and the launch. Returns (output,
+    cu_seqlens_q values, cu_seqlens_k values), or None with nothing launched."""
+    if type(max_seqlen_q) is not int or max_seqlen_q != 1 or type(max_seqlen_k) is not int:
+        return None
+    op = native.torch_op() if q.is_cuda and native.USE_TORCH_OP else None
+    if op is None:
+        return None
+    offsets = op.PackedOffsets()
+    out = op.contiguous_decode(q, k, v, scale, False, max_seqlen_k, cu_seqlens_q, cu_seqlens_k,
+                               offsets=offsets)
+    return None if out is None else (out, *offsets.get())
+
+
 def route_varlen(q, k, v, cu_seqlens_k: torch.Tensor, q_offsets: list[int], k_offsets: list[int],
                  max_seqlen_k: int, scale, causal,
-                 cu_seqlens_q: torch.Tensor | None = None) -> DecodeRoute:
+                 cu_seqlens_q: torch.Tensor | None = None,
+                 started: torch.Tensor | None = None) -> DecodeRoute:
     """Packed decode: sequence b's keys are rows [cu_k[b], cu_k[b+1]) of k/v,
-    read in place (first rows and lengths come from the offsets on the device)."""
+    read in place (first rows and lengths come from the offsets on the device).
+    ``started``: the output of a start_varlen launch of this call."""
     reason = _common_reason(q, k.shape[1], q.shape[-1])
     if reason is not None:
         return DecodeRoute(reason)
@@ -193,6 +214,8 @@ def route_varlen(q, k, v, cu_seqlens_k: torch.Tensor, q_offsets: list[int], k_of
         return DecodeRoute(reason)
 
     def run() -> torch.Tensor:
+        if started is not None:
+            return started
         if cu_seqlens_q is not None:
             result = _contiguous(q, k, v, scale, False, width, cu_seqlens_q, cu_seqlens_k)
             if result is not None:

@@ -90,14 +90,17 @@ def validate_cumulative_lengths(
     max_seqlen: int,
     name: str,
     require_non_empty: bool = False,
+    values: list[int] | None = None,
 ) -> list[int]:
     """Host copy of a cumulative-length vector after checking it
-    (mxflashattn/validation.py:79-100). Reads the tensor back to the host."""
+    (mxflashattn/validation.py:79-100). Reads the tensor back to the host,
+    unless the caller has its ``values`` there already."""
     if not isinstance(cu_seqlens, torch.Tensor) or cu_seqlens.ndim != 1:
         raise TypeError(f"{name} must be a one-dimensional torch.Tensor")
     if cu_seqlens.dtype not in (torch.int32, torch.int64):
         raise TypeError(f"{name} must use int32 or int64")
-    values = [int(x) for x in cu_seqlens.detach().cpu().tolist()]
+    if values is None:
+        values = [int(x) for x in cu_seqlens.detach().cpu().tolist()]
     if len(values) < 2 or values[0] != 0 or values[-1] != total_tokens:
         raise ValueError(f"{name} must start at zero and cover all tokens")
     steps = [right - left for left, right in zip(values, values[1:])]

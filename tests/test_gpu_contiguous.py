@@ -118,3 +118,30 @@ def test_offsets_that_name_no_keys_read_nothing_outside(device):
             q[b:b + 1].float().cpu(), k[a:e].float().cpu(), v[a:e].float().cpu(),
             softmax_scale=0.125)[0]
         close(out[b], want, torch.float16)
+
+
+def test_packed_offsets_are_checked_after_the_launch(device):
+    """Offsets the API rejects raise the same errors as before the kernels
+    went out first, leave the next call right, and name no row outside."""
+    k, v = (randn(60, 2, 64, dtype=torch.float16, seed=s).to(device) for s in (8, 9))
+    q = randn(3, 4, 64, dtype=torch.float16, seed=10).to(device)
+    good = torch.tensor([0, 20, 21, 60])
+
+    def call(cu_q, cu_k, max_q=1, max_k=60):
+        return mx.flash_attn_varlen_func(q, k, v, torch.tensor(cu_q).to(device),
+                                         torch.as_tensor(cu_k).to(device), max_q, max_k)
+
+    for cu_q, cu_k, match in (([0, 1, 2, 3], [0, 20, 70, 60], "cu_seqlens_k must be monotonically"),
+                              ([0, 1, 2, 3], [0, 20, 20, 60], "must be non-empty"),
+                              ([0, 1, 2, 3], [0, 20, 21, 59], "cu_seqlens_k must start at zero"),
+                              ([0, 2, 2, 3], good, "cu_seqlens_q contains a sequence longer"),
+                              ([1, 1, 2, 3], good, "cu_seqlens_q must start at zero"),
+                              ([0, 1, 2, 3, 3], good, "same batch size")):
+        with pytest.raises(ValueError, match=match):
+            call(cu_q, cu_k)
+    with pytest.raises(ValueError, match="cu_seqlens_k contains a sequence longer"):
+        call([0, 1, 2, 3], good, max_k=38)
+    out = call([0, 1, 2, 3], good)
+    ref = reference_port.attention_varlen(q.float().cpu(), k.float().cpu(), v.float().cpu(),
+                                          [0, 1, 2, 3], good.tolist(), softmax_scale=0.125)
+    close(out, ref, torch.float16)
