@@ -1,6 +1,7 @@
 // Host-side torch operator in front of the C ABI (include/mxfa_mi355x.h): the
-// hot decode call and the vLLM-form page append without Python's
-// per-argument marshalling.
+// decode calls and the cache writes without Python's per-argument marshalling
+// (a call of several query tokens, an fp8 cache or options took 17-30 us of
+// host time through ctypes, an append about 12; small calls were bound by it).
 //
 // decode(q, k_cache, v_cache, block_table, cache_seqlens, scale, out,
 //        num_splits, seqlen_add) takes the common call (one query
@@ -9,7 +10,8 @@
 // launches it on torch's current HIP stream and returns the output.
 // num_splits None is mxfa_split_heuristic's choice. For any
 // other call it launches nothing and returns None; the Python binding then
-// takes the call and gives its usual errors.
+// takes the call and gives its usual errors. decode_tokens (the general call),
+// contiguous_decode, reshape_and_cache and append_kv below do the same.
 //
 // The workspace is grow-only per (device, stream): a buffer replaced by a
 // larger one stays alive until the process ends, since a HIP graph captured
@@ -388,47 +390,267 @@ py::object contiguous_decode(const at::Tensor &q, const at::Tensor &k, const at:
   return py::cast(out);
 }
 
-// reshape_and_cache(key, value, key_cache, value_cache, slot_mapping): the
-// vLLM-form append of 16-bit caches (mxfa_reshape_and_cache_launch) for the
-// common call: key/value [T, HKV, HD] sharing strides with a contiguous last
-// dim, caches [pages, PS, HKV, HD] of their dtype sharing strides, int64
-// contiguous slots (at least T of them), every tensor on the current GPU.
-// Returns true once launched on torch's current stream; false (nothing
-// launched) for any other call, which the Python binding then takes.
-bool reshape_and_cache(const at::Tensor &key, const at::Tensor &value,
-                       const at::Tensor &key_cache, const at::Tensor &value_cache,
-                       const at::Tensor &slot_mapping) {
-  const at::ScalarType dt = key.scalar_type();
-  if (dt != at::kHalf && dt != at::kBFloat16) return false;
-  if (!key.is_cuda() || value.scalar_type() != dt || key_cache.scalar_type() != dt ||
-      value_cache.scalar_type() != dt || slot_mapping.scalar_type() != at::kLong)
+// A float32 [n] vector's address (sinks, ALiBi slopes), null for none; false
+// for a tensor the kernels do not read in place.
+bool head_vector(const c10::optional<at::Tensor> &t, int64_t n, const at::Device &device,
+                 const float *&ptr) {
+  ptr = nullptr;
+  if (!t.has_value()) return true;
+  if (t->scalar_type() != at::kFloat || t->device() != device || t->dim() != 1 ||
+      t->size(0) != n || !t->is_contiguous())
     return false;
-  if (key.dim() != 3 || !value.sizes().equals(key.sizes()) || !value.strides().equals(key.strides()) ||
-      key.stride(2) != 1)
+  ptr = t->data_ptr<float>();
+  return true;
+}
+
+// A per-tensor scale's address (one float32, or one broadcast), null for none.
+bool tensor_scale(const c10::optional<at::Tensor> &t, const at::Device &device,
+                  const float *&ptr) {
+  ptr = nullptr;
+  if (!t.has_value()) return true;
+  if (t->scalar_type() != at::kFloat || t->device() != device || t->numel() < 1) return false;
+  if (t->numel() != 1)
+    for (const int64_t st : t->strides())
+      if (st != 0) return false;
+  ptr = t->data_ptr<float>();
+  return true;
+}
+
+// decode_tokens(q, k_cache, v_cache, block_table, cache_seqlens, scale, out,
+// num_splits, seqlen_add, causal, window_left, softcap, k_scale, v_scale, sinks,
+// alibi_slopes): the general paged call (several query tokens, fp8 caches,
+// window, soft cap, sinks, ALiBi) with tensors the kernels read in place; a
+// causal query of more columns than one launch takes runs as several. Returns
+// the output, or None (nothing launched) for any other call, which the Python
+// binding then takes.
+py::object decode_tokens(const at::Tensor &q, const at::Tensor &k_cache, const at::Tensor &v_cache,
+                         const at::Tensor &block_table, const at::Tensor &cache_seqlens,
+                         double scale, const c10::optional<at::Tensor> &out_arg,
+                         const c10::optional<int64_t> &num_splits_arg, int64_t seqlen_add,
+                         bool causal, int64_t window_left, double softcap,
+                         const c10::optional<at::Tensor> &k_scale,
+                         const c10::optional<at::Tensor> &v_scale,
+                         const c10::optional<at::Tensor> &sinks,
+                         const c10::optional<at::Tensor> &alibi_slopes) {
+  const at::ScalarType dt = q.scalar_type();
+  const bool fp8 = k_cache.scalar_type() == at::kFloat8_e4m3fn;
+  if ((dt != at::kHalf && dt != at::kBFloat16) || (!fp8 && k_cache.scalar_type() != dt) ||
+      v_cache.scalar_type() != k_cache.scalar_type())
+    return py::none();
+  if (!q.is_cuda() || (q.dim() != 3 && q.dim() != 4) || q.stride(-1) != 1) return py::none();
+  if (k_cache.dim() != 4 || !v_cache.sizes().equals(k_cache.sizes()) ||
+      !v_cache.strides().equals(k_cache.strides()) || k_cache.stride(3) != 1)
+    return py::none();
+  if (block_table.scalar_type() != at::kInt || cache_seqlens.scalar_type() != at::kInt ||
+      block_table.dim() != 2 || block_table.stride(1) != 1 || cache_seqlens.dim() != 1 ||
+      !cache_seqlens.is_contiguous())
+    return py::none();
+  const at::Device device = q.device();
+  if (k_cache.device() != device || v_cache.device() != device ||
+      block_table.device() != device || cache_seqlens.device() != device ||
+      device.index() != c10::hip::current_device())
+    return py::none();
+  const int64_t batch = q.size(0), ql = q.dim() == 4 ? q.size(1) : 1;
+  const int64_t hq = q.size(-2), hd = q.size(-1);
+  const int64_t pages = k_cache.size(0), ps = k_cache.size(1), hkv = k_cache.size(2);
+  if (batch < 1 || ql < 1 || hkv < 1 || ps < 1 || hq % hkv || hq / hkv > 16 || hq < hkv ||
+      k_cache.size(3) != hd || block_table.size(0) != batch || cache_seqlens.size(0) != batch ||
+      block_table.size(1) < 1)
+    return py::none();
+  const int64_t limit = std::numeric_limits<int>::max() / 64;
+  if (batch > limit || hq > limit || ql > limit || pages > std::numeric_limits<int>::max() ||
+      ps > 4096 || block_table.size(1) > std::numeric_limits<int>::max())
+    return py::none();
+  const int64_t gq = hq / hkv;
+  if ((ql * gq > 16 && !causal) || window_left < -1 || window_left > 1 << 30 ||
+      !(softcap >= 0.0) || softcap == std::numeric_limits<double>::infinity())
+    return py::none();
+  if (seqlen_add < -(1 << 29) || seqlen_add > 1 << 30) return py::none();
+  const float *ks, *vs, *sink_ptr, *alibi_ptr;
+  if (!head_vector(sinks, hq, device, sink_ptr) || !head_vector(alibi_slopes, hq, device, alibi_ptr))
+    return py::none();
+  if (!tensor_scale(fp8 ? k_scale : c10::nullopt, device, ks) ||
+      !tensor_scale(fp8 ? v_scale : c10::nullopt, device, vs))
+    return py::none();
+  // Strides (batch, token, head); the token stride of one token is not used.
+  const auto strides = [&](const at::Tensor &t, int64_t (&s)[3]) {
+    s[0] = t.stride(0);
+    s[1] = ql > 1 ? t.stride(1) : 0;
+    s[2] = t.stride(-2);
+  };
+  int64_t qs[3], os[3];
+  strides(q, qs);
+  if (!aligned(q.data_ptr(), 16) || ((qs[0] | qs[1] | qs[2]) & 7) || (hq > 1 && qs[2] < hd))
+    return py::none();
+  at::Tensor out;
+  if (out_arg.has_value()) {
+    out = *out_arg;
+    if (out.scalar_type() != dt || out.device() != device || !out.sizes().equals(q.sizes()) ||
+        out.stride(-1) != 1 || at::has_internal_overlap(out) == at::MemOverlap::Yes)
+      return py::none();
+    strides(out, os);
+    if (!aligned(out.data_ptr(), 8) || ((os[0] | os[1] | os[2]) & 3)) return py::none();
+  } else {
+    out = at::empty(q.sizes(), q.options());
+    strides(out, os);
+  }
+  const bool extras = window_left >= 0 || softcap > 0 || sink_ptr || alibi_ptr;
+  const int width = (int)block_table.size(1), cus = num_cus(device.index());
+  const int64_t wide = mxfa_package_launch_columns((int)hd, (int)ps, fp8, extras);
+  const auto heuristic = [&](int64_t columns, int &ns) {
+    const auto f = fp8 ? mxfa_split_heuristic_fp8 : mxfa_split_heuristic;
+    return f((int)batch, (int)(hkv * columns), (int)hkv, (int)hd, (int)ps, width, cus, &ns) ==
+           MXFA_OK;
+  };
+  // num_splits as the Python binding's default_num_splits chooses it: asked for
+  // the columns of one launch, then, past 16 of them and unless the
+  // per-sequence kernel was picked, for a launch of several column groups.
+  int ns = 0;
+  if (num_splits_arg.has_value()) {
+    const int64_t v = *num_splits_arg;
+    if ((v <= 0 && v != MXFA_SPLITS_PER_SEQUENCE) || v > 65535) return py::none();
+    ns = (int)v;
+  } else {
+    if (!heuristic(gq * std::min<int64_t>(ql, 16 / gq), ns)) return py::none();
+    if (ql > 16 / gq && ns != MXFA_SPLITS_PER_SEQUENCE && wide > 16 && !heuristic(17, ns))
+      return py::none();
+  }
+  // Tokens per launch (native.tokens_per_launch).
+  const int64_t columns = ql * gq > 16 && ns != MXFA_SPLITS_PER_SEQUENCE ? wide : 16;
+  int64_t tokens = std::min<int64_t>(ql, columns / gq);
+  if (columns > 16) {
+    const int64_t launches = (ql + tokens - 1) / tokens;
+    tokens = (ql + launches - 1) / launches;
+  }
+  size_t ws_bytes = 0;
+  if (mxfa_split_decode_workspace_size((int)batch, (int)(hq * tokens), (int)hd, ns, &ws_bytes) !=
+      MXFA_OK)
+    return py::none();
+  void *stream = (void *)c10::hip::getCurrentHIPStream(device.index()).stream();
+  at::Tensor ws_t;
+  if (ws_bytes) ws_t = workspace(device, stream, ws_bytes);
+  void *ws = ws_bytes ? ws_t.data_ptr() : nullptr;
+  poison(stream, out, ws_bytes ? &ws_t : nullptr);
+  const int64_t esz = 2;
+  for (int64_t t = 0; t < ql; t += tokens) {
+    const int64_t n = std::min(tokens, ql - t);
+    // Tokens [t, t + n) as the last n tokens of sequences shortened by the
+    // tokens after them.
+    const int rc = mxfa_package_decode_tokens_launch(
+        (const char *)q.data_ptr() + t * qs[1] * esz, qs[0], qs[1], qs[2], (int)n, causal,
+        (int)window_left, sink_ptr, (float)softcap, alibi_ptr, k_cache.data_ptr(),
+        v_cache.data_ptr(), k_cache.stride(0), k_cache.stride(1), k_cache.stride(2),
+        block_table.data_ptr<int32_t>(), block_table.stride(0),
+        cache_seqlens.data_ptr<int32_t>(), (int)(seqlen_add - (ql - t - n)),
+        (char *)out.data_ptr() + t * os[1] * esz, os[0], os[1], os[2], ws, ws_bytes, (float)scale,
+        (int)batch, (int)hq, (int)hkv, (int)hd, (int)ps, width, (int)pages,
+        dt == at::kBFloat16 ? MXFA_DTYPE_BF16 : MXFA_DTYPE_F16,
+        fp8                  ? MXFA_DTYPE_FP8_E4M3
+        : dt == at::kBFloat16 ? MXFA_DTYPE_BF16
+                              : MXFA_DTYPE_F16,
+        ks, vs, ns, stream);
+    if (t == 0 && (rc == MXFA_EUNSUPPORTED || rc == MXFA_EINVAL))
+      return py::none();  // nothing launched
+    if (rc != MXFA_OK)
+      throw std::runtime_error(std::string("mxfa_split_decode_multi_launch failed (") +
+                               std::to_string(rc) + "): " + mxfa_strerror(rc));
+  }
+  return py::cast(out);
+}
+
+// Source rows K and V (of `rank` dims) sharing strides with a contiguous last
+// dim, and paged caches sharing theirs, all on the current GPU; cache_dt the
+// caches' type.
+bool append_tensors(const at::Tensor &key, const at::Tensor &value, const at::Tensor &key_cache,
+                    const at::Tensor &value_cache, int64_t rank, at::ScalarType cache_dt) {
+  const at::ScalarType dt = key.scalar_type();
+  if ((dt != at::kHalf && dt != at::kBFloat16) || !key.is_cuda() || value.scalar_type() != dt ||
+      key_cache.scalar_type() != cache_dt || value_cache.scalar_type() != cache_dt)
+    return false;
+  if (key.dim() != rank || !value.sizes().equals(key.sizes()) ||
+      !value.strides().equals(key.strides()) || key.stride(-1) != 1)
     return false;
   if (key_cache.dim() != 4 || !value_cache.sizes().equals(key_cache.sizes()) ||
       !value_cache.strides().equals(key_cache.strides()) || key_cache.stride(3) != 1)
     return false;
-  if (key.size(1) != key_cache.size(2) || key.size(2) != key_cache.size(3)) return false;
-  if (slot_mapping.dim() != 1 || !slot_mapping.is_contiguous() ||
-      slot_mapping.size(0) < key.size(0))
+  if (key.size(-2) != key_cache.size(2) || key.size(-1) != key_cache.size(3)) return false;
+  const at::Device device = key.device();
+  return value.device() == device && key_cache.device() == device &&
+         value_cache.device() == device && device.index() == c10::hip::current_device();
+}
+
+// reshape_and_cache(key, value, key_cache, value_cache, slot_mapping, k_scale,
+// v_scale): the vLLM-form append, 16-bit (mxfa_reshape_and_cache_launch) or
+// into fp8 caches (mxfa_reshape_and_cache_fp8_launch), for the common call:
+// key/value [T, HKV, HD], caches [pages, PS, HKV, HD], int64 contiguous slots
+// (at least T of them), scales None or float32 device tensors.
+// Returns true once launched on torch's current stream; false (nothing
+// launched) for any other call, which the Python binding then takes.
+bool reshape_and_cache(const at::Tensor &key, const at::Tensor &value,
+                       const at::Tensor &key_cache, const at::Tensor &value_cache,
+                       const at::Tensor &slot_mapping, const c10::optional<at::Tensor> &k_scale,
+                       const c10::optional<at::Tensor> &v_scale) {
+  const at::ScalarType dt = key.scalar_type();
+  const bool fp8 = key_cache.scalar_type() == at::kFloat8_e4m3fn;
+  if (!append_tensors(key, value, key_cache, value_cache, 3, fp8 ? at::kFloat8_e4m3fn : dt))
     return false;
   const at::Device device = key.device();
-  if (value.device() != device || key_cache.device() != device ||
-      value_cache.device() != device || slot_mapping.device() != device ||
-      device.index() != c10::hip::current_device())
+  if (slot_mapping.scalar_type() != at::kLong || slot_mapping.dim() != 1 ||
+      !slot_mapping.is_contiguous() || slot_mapping.size(0) < key.size(0) ||
+      slot_mapping.device() != device)
+    return false;
+  const float *ks, *vs;
+  if (!tensor_scale(fp8 ? k_scale : c10::nullopt, device, ks) ||
+      !tensor_scale(fp8 ? v_scale : c10::nullopt, device, vs))
     return false;
   void *stream = (void *)c10::hip::getCurrentHIPStream(device.index()).stream();
-  const int rc = mxfa_reshape_and_cache_launch(
-      key.data_ptr(), value.data_ptr(), key.stride(0), key.stride(1), key_cache.data_ptr(),
-      value_cache.data_ptr(), key_cache.stride(0), key_cache.stride(1), key_cache.stride(2),
-      slot_mapping.data_ptr<int64_t>(), (int)key.size(0), (int)key.size(1), (int)key.size(2),
-      (int)key_cache.size(1), (int)key_cache.size(0),
-      dt == at::kBFloat16 ? MXFA_DTYPE_BF16 : MXFA_DTYPE_F16, stream);
+  const int code = dt == at::kBFloat16 ? MXFA_DTYPE_BF16 : MXFA_DTYPE_F16;
+  const int rc =
+      fp8 ? mxfa_reshape_and_cache_fp8_launch(
+                key.data_ptr(), value.data_ptr(), key.stride(0), key.stride(1),
+                key_cache.data_ptr(), value_cache.data_ptr(), key_cache.stride(0),
+                key_cache.stride(1), key_cache.stride(2), slot_mapping.data_ptr<int64_t>(),
+                (int)key.size(0), (int)key.size(1), (int)key.size(2), (int)key_cache.size(1),
+                (int)key_cache.size(0), code, ks, vs, stream)
+          : mxfa_reshape_and_cache_launch(
+                key.data_ptr(), value.data_ptr(), key.stride(0), key.stride(1),
+                key_cache.data_ptr(), value_cache.data_ptr(), key_cache.stride(0),
+                key_cache.stride(1), key_cache.stride(2), slot_mapping.data_ptr<int64_t>(),
+                (int)key.size(0), (int)key.size(1), (int)key.size(2), (int)key_cache.size(1),
+                (int)key_cache.size(0), code, stream);
   if (rc == MXFA_EUNSUPPORTED || rc == MXFA_EINVAL) return false;  // nothing launched
   if (rc != MXFA_OK)
     throw std::runtime_error(std::string("mxfa_reshape_and_cache_launch failed (") +
                              std::to_string(rc) + "): " + mxfa_strerror(rc));
+  return true;
+}
+
+// append_kv(k, v, k_cache, v_cache, block_table, cache_seqlens): the table-form
+// append (mxfa_append_kv_launch) of 16-bit rows [B, S, HKV, HD], int32 table and
+// lengths. True once launched, false (nothing launched) for any other call.
+bool append_kv(const at::Tensor &k, const at::Tensor &v, const at::Tensor &k_cache,
+               const at::Tensor &v_cache, const at::Tensor &block_table,
+               const at::Tensor &cache_seqlens) {
+  if (!append_tensors(k, v, k_cache, v_cache, 4, k.scalar_type())) return false;
+  const at::Device device = k.device();
+  if (block_table.scalar_type() != at::kInt || cache_seqlens.scalar_type() != at::kInt ||
+      block_table.dim() != 2 || block_table.stride(1) != 1 || cache_seqlens.dim() != 1 ||
+      !cache_seqlens.is_contiguous() || block_table.device() != device ||
+      cache_seqlens.device() != device || block_table.size(0) != k.size(0) ||
+      block_table.size(1) < 1 || cache_seqlens.size(0) != k.size(0))
+    return false;
+  void *stream = (void *)c10::hip::getCurrentHIPStream(device.index()).stream();
+  const int rc = mxfa_append_kv_launch(
+      k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1), k.stride(2), k_cache.data_ptr(),
+      v_cache.data_ptr(), k_cache.stride(0), k_cache.stride(1), k_cache.stride(2),
+      block_table.data_ptr<int32_t>(), block_table.stride(0), cache_seqlens.data_ptr<int32_t>(),
+      (int)k.size(0), (int)k.size(1), (int)k.size(2), (int)k.size(3), (int)k_cache.size(1),
+      (int)block_table.size(1), (int)k_cache.size(0),
+      k.scalar_type() == at::kBFloat16 ? MXFA_DTYPE_BF16 : MXFA_DTYPE_F16, stream);
+  if (rc == MXFA_EUNSUPPORTED || rc == MXFA_EINVAL) return false;  // nothing launched
+  if (rc != MXFA_OK)
+    throw std::runtime_error(std::string("mxfa_append_kv_launch failed (") + std::to_string(rc) +
+                             "): " + mxfa_strerror(rc));
   return true;
 }
 
@@ -446,8 +668,16 @@ PYBIND11_MODULE(_mxfa_torch, m) {
         py::arg("cu_seqlens_q") = py::none(), py::arg("cu_seqlens_k") = py::none(),
         py::arg("seqlens") = py::none(), py::arg("out") = py::none(),
         py::arg("offsets") = py::none());
+  m.def("decode_tokens", &decode_tokens, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
+        py::arg("block_table"), py::arg("cache_seqlens"), py::arg("scale"), py::arg("out"),
+        py::arg("num_splits"), py::arg("seqlen_add"), py::arg("causal"), py::arg("window_left"),
+        py::arg("softcap"), py::arg("k_scale"), py::arg("v_scale"), py::arg("sinks"),
+        py::arg("alibi_slopes"));
   m.def("reshape_and_cache", &reshape_and_cache, py::arg("key"), py::arg("value"),
-        py::arg("key_cache"), py::arg("value_cache"), py::arg("slot_mapping"));
+        py::arg("key_cache"), py::arg("value_cache"), py::arg("slot_mapping"),
+        py::arg("k_scale") = py::none(), py::arg("v_scale") = py::none());
+  m.def("append_kv", &append_kv, py::arg("k"), py::arg("v"), py::arg("k_cache"),
+        py::arg("v_cache"), py::arg("block_table"), py::arg("cache_seqlens"));
   m.def("abi_version", &mxfa_abi_version);
   m.def("workspace_bytes", &workspace_bytes,
         "(bytes of live workspaces, bytes of workspaces replaced by larger ones)");

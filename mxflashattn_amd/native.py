@@ -630,6 +630,12 @@ def default_num_splits(q: torch.Tensor, k_cache: torch.Tensor, block_table: torc
     return ns
 
 
+def _op_scales(*values) -> bool:
+    """Scales, sinks and slopes as the operator takes them: tensors or None
+    (Python floats become cached device scalars in the binding)."""
+    return all(v is None or isinstance(v, torch.Tensor) for v in values)
+
+
 def paged_decode_split(
     q: torch.Tensor,
     k_cache: torch.Tensor,
@@ -672,17 +678,25 @@ def paged_decode_split(
     the one-launch per-sequence kernel (default: split_heuristic, which picks
     the latter for batches of short sequences by the block table's capacity).
     """
-    if (USE_TORCH_OP and k_scale is None and v_scale is None and window_left < 0
-            and sinks is None and softcap == 0 and alibi_slopes is None
-            and (q.dim() == 3 or q.shape[1] == 1)):
+    if USE_TORCH_OP:
+        # The operator takes the common calls (one 16-bit token, then the
+        # general form) and hands any other back as None.
         op = torch_op()
         if op is not None:
-            result = op.decode(q, k_cache, v_cache, block_table, cache_seqlens,
-                               float(softmax_scale), out,
-                               None if num_splits is None else int(num_splits),
-                               int(seqlen_add))
+            result = None
+            ns = None if num_splits is None else int(num_splits)
+            if (k_scale is None and v_scale is None and window_left < 0 and sinks is None
+                    and softcap == 0 and alibi_slopes is None
+                    and (q.dim() == 3 or q.shape[1] == 1)):
+                result = op.decode(q, k_cache, v_cache, block_table, cache_seqlens,
+                                   float(softmax_scale), out, ns, int(seqlen_add))
+            if result is None and _op_scales(k_scale, v_scale, sinks, alibi_slopes):
+                result = op.decode_tokens(q, k_cache, v_cache, block_table, cache_seqlens,
+                                          float(softmax_scale), out, ns, int(seqlen_add),
+                                          bool(causal), int(window_left), float(softcap),
+                                          k_scale, v_scale, sinks, alibi_slopes)
             if result is not None:
-                return result
+                return result if out is None else out
     if out is not None and (out.data_ptr() % 8 or any(st % 4 for st in out.stride()[:-1])):
         # The kernels store 8-byte pieces of each output row; a view that is
         # not laid out for that gets the result through a packed copy.
@@ -886,13 +900,17 @@ def reshape_and_cache(
 
     float8_e4m3fn caches store e4m3fn_rne(saturate(x / scale)) with the
     per-tensor k_scale / v_scale; 16-bit caches are a bit-exact copy."""
-    if USE_TORCH_OP and k_scale is None and v_scale is None:
+    if USE_TORCH_OP:
         op = torch_op()
-        # The common 16-bit call goes through the C++ operator; it launches
-        # nothing and returns False for any other call, taken below.
-        if op is not None and op.reshape_and_cache(key, value, key_cache, value_cache,
-                                                   slot_mapping):
-            return
+        # The common call goes through the C++ operator; it launches nothing
+        # and returns False for any other call, taken below.
+        if op is not None:
+            if k_scale is None and v_scale is None:
+                if op.reshape_and_cache(key, value, key_cache, value_cache, slot_mapping):
+                    return
+            elif _op_scales(k_scale, v_scale) and op.reshape_and_cache(
+                    key, value, key_cache, value_cache, slot_mapping, k_scale, v_scale):
+                return
     if key.dim() != 3 or value.shape != key.shape:
         raise ValueError("key/value must be [num_tokens, kv_heads, head_dim]")
     if key_cache.dim() != 4 or value_cache.shape != key_cache.shape:
@@ -939,6 +957,10 @@ def append_kv(
     cache_seqlens: torch.Tensor,
 ) -> None:
     """Block-table append: k[b, t] -> position cache_seqlens[b] + t (seqlens unchanged)."""
+    if USE_TORCH_OP:
+        op = torch_op()
+        if op is not None and op.append_kv(k, v, k_cache, v_cache, block_table, cache_seqlens):
+            return
     if k.dim() != 4 or v.shape != k.shape:
         raise ValueError("k/v must be [batch, new_tokens, kv_heads, head_dim]")
     if k_cache.dim() != 4 or v_cache.shape != k_cache.shape:
