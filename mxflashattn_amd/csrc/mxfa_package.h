@@ -19,7 +19,9 @@ int mxfa_package_launch_columns(int head_dim, int page_size, int fp8, int extras
 // mxfa_split_decode_multi_launch (same arguments, checks and results) for up
 // to mxfa_package_launch_columns columns: every 16 columns past the first are
 // another column group of the same wave, so the keys are read once for all.
-// With num_splits = MXFA_SPLITS_PER_SEQUENCE at most 16 columns.
+// With num_splits = MXFA_SPLITS_PER_SEQUENCE at most 16 columns. advance (int32
+// [batch], or null) is moved on by advance_by once the call has read the
+// lengths; it may be seqlens itself.
 int mxfa_package_decode_tokens_launch(
     const void *q, int64_t q_stride_b, int64_t q_stride_t, int64_t q_stride_h, int q_len,
     int causal, int window_left, const float *sinks, float softcap, const float *alibi_slopes,
@@ -29,7 +31,7 @@ int mxfa_package_decode_tokens_launch(
     int64_t out_stride_t, int64_t out_stride_h, void *workspace, size_t workspace_bytes,
     float scale, int batch, int q_heads, int kv_heads, int head_dim, int page_size,
     int block_table_width, int num_pages, int dtype, int kv_dtype, const float *k_scale,
-    const float *v_scale, int num_splits, void *stream);
+    const float *v_scale, int num_splits, int32_t *advance, int advance_by, void *stream);
 
 // Decode over keys that lie in consecutive rows, read in place (16-bit caches):
 // k and v rows of kv head h at first_stride * first(b) + token_stride * i +

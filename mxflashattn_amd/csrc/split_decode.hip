@@ -138,6 +138,8 @@ struct SplitArgs {
   const float *alibi;  // per query head ALiBi slopes, nullptr: none
   int min_seqlen_add;  // 0, or -2^30 where lengths below zero count as 0
   int max_cols;        // columns (query tokens x heads per kv head) the entry point takes
+  int32_t *advance;    // lengths to move on by advance_by once they are read (null: none)
+  int advance_by;
   bool contiguous;     // a sequence's keys are consecutive rows: one page per sequence (ps 1,
                        // btw = the longest sequence, bt = its first row or page, bt_stride 1)
 };
@@ -337,7 +339,7 @@ static void combine_shape(int batch, int hq, int hd, int num_splits, CombinePara
 static int launch_combine(void *ws, void *out, const float *sinks, int64_t o_sb, int64_t o_st,
                           int64_t o_sh,
                           int batch, int hq, int hkv, int ql, int hd, int dtype, int ns,
-                          hipStream_t st) {
+                          int32_t *advance, int advance_by, hipStream_t st) {
   const WsLayout w = ws_layout(batch, hq * ql, hd, ns);
   CombineParams c;
   c.ws_o = (const float *)ws;
@@ -354,6 +356,8 @@ static int launch_combine(void *ws, void *out, const float *sinks, int64_t o_sb,
   c.num_ranges = ns;
   combine_shape(batch, hq * ql, hd, ns, c);
   c.sinks = sinks;
+  c.advance = advance;
+  c.advance_by = advance_by;
 #ifdef MXFA_WAVE_STAMPS
   c.stamps = g_wave_stamps ? g_wave_stamps + kStampCombineBase : nullptr;
 #endif
@@ -413,6 +417,8 @@ static SplitArgs split_args(const void *q, int64_t q_stride_b, int64_t q_stride_
   a.alibi = nullptr;
   a.min_seqlen_add = 0;
   a.max_cols = kMaxCols;
+  a.advance = nullptr;
+  a.advance_by = 0;
   a.contiguous = false;
   return a;
 }
@@ -441,14 +447,26 @@ static int launch_seq(const SplitArgs &a, hipStream_t st) {
   }
 }
 
+// Lengths moved on after the per-sequence kernel, which has no second launch.
+__global__ __launch_bounds__(256) void advance_kernel(int32_t *seqlens, int n, int by) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) seqlens[i] += by;
+}
+
 static int run_split(const SplitArgs &a, bool with_combine, hipStream_t st) {
   int rc = check_split_args(a);
   if (rc != MXFA_OK) return rc;
-  if (a.num_splits == MXFA_SPLITS_PER_SEQUENCE) return launch_seq(a, st);
+  if (a.num_splits == MXFA_SPLITS_PER_SEQUENCE) {
+    rc = launch_seq(a, st);
+    if (rc != MXFA_OK || !a.advance) return rc;
+    hipLaunchKernelGGL(advance_kernel, dim3((a.batch + 255) / 256), dim3(256), 0, st, a.advance,
+                       a.batch, a.advance_by);
+    return hipGetLastError() == hipSuccess ? MXFA_OK : MXFA_ELAUNCH;
+  }
   rc = launch_partial(a, st);
   if (rc != MXFA_OK || !with_combine) return rc;
   return launch_combine(a.ws, a.out, a.sinks, a.o_sb, a.o_st, a.o_sh, a.batch, a.hq, a.hkv,
-                        a.ql, a.hd, a.dtype, a.num_splits, st);
+                        a.ql, a.hd, a.dtype, a.num_splits, a.advance, a.advance_by, st);
 }
 
 static SplitArgs fp8_args(SplitArgs a, const float *k_scale, const float *v_scale) {
@@ -764,7 +782,7 @@ int mxfa_split_decode_combine_launch(void *workspace, size_t workspace_bytes, vo
     return MXFA_EWORKSPACE;
   return launch_combine(workspace, out, nullptr, out_stride_b, 0, out_stride_h, batch, q_heads,
                         kv_heads,
-                        1, head_dim, dtype, num_splits, (hipStream_t)stream);
+                        1, head_dim, dtype, num_splits, nullptr, 0, (hipStream_t)stream);
 }
 
 int mxfa_split_decode_multi_launch(
@@ -791,8 +809,11 @@ int mxfa_package_decode_tokens_launch(
     int64_t out_stride_t, int64_t out_stride_h, void *workspace, size_t workspace_bytes,
     float scale, int batch, int q_heads, int kv_heads, int head_dim, int page_size,
     int block_table_width, int num_pages, int dtype, int kv_dtype, const float *k_scale,
-    const float *v_scale, int num_splits, void *stream) {
-  return run_tokens(split_args(MXFA_SPLIT_ARGS), q_stride_t, q_len, causal, window_left, sinks,
+    const float *v_scale, int num_splits, int32_t *advance, int advance_by, void *stream) {
+  SplitArgs a = split_args(MXFA_SPLIT_ARGS);
+  a.advance = advance;
+  a.advance_by = advance_by;
+  return run_tokens(a, q_stride_t, q_len, causal, window_left, sinks,
                     softcap, alibi_slopes, out_stride_t, kv_dtype, k_scale, v_scale, true,
                     (hipStream_t)stream);
 }

@@ -420,7 +420,8 @@ bool tensor_scale(const c10::optional<at::Tensor> &t, const at::Device &device,
 // num_splits, seqlen_add, causal, window_left, softcap, k_scale, v_scale, sinks,
 // alibi_slopes): the general paged call (several query tokens, fp8 caches,
 // window, soft cap, sinks, ALiBi) with tensors the kernels read in place; a
-// causal query of more columns than one launch takes runs as several. Returns
+// causal query of more columns than one launch takes runs as several.
+// cache_seqlens moves on by `advance` once it has been read. Returns
 // the output, or None (nothing launched) for any other call, which the Python
 // binding then takes.
 py::object decode_tokens(const at::Tensor &q, const at::Tensor &k_cache, const at::Tensor &v_cache,
@@ -431,7 +432,7 @@ py::object decode_tokens(const at::Tensor &q, const at::Tensor &k_cache, const a
                          const c10::optional<at::Tensor> &k_scale,
                          const c10::optional<at::Tensor> &v_scale,
                          const c10::optional<at::Tensor> &sinks,
-                         const c10::optional<at::Tensor> &alibi_slopes) {
+                         const c10::optional<at::Tensor> &alibi_slopes, int64_t advance) {
   const at::ScalarType dt = q.scalar_type();
   const bool fp8 = k_cache.scalar_type() == at::kFloat8_e4m3fn;
   if ((dt != at::kHalf && dt != at::kBFloat16) || (!fp8 && k_cache.scalar_type() != dt) ||
@@ -465,6 +466,7 @@ py::object decode_tokens(const at::Tensor &q, const at::Tensor &k_cache, const a
   if ((ql * gq > 16 && !causal) || window_left < -1 || window_left > 1 << 30 ||
       !(softcap >= 0.0) || softcap == std::numeric_limits<double>::infinity())
     return py::none();
+  if (advance < 0 || advance > 1 << 30) return py::none();
   if (seqlen_add < -(1 << 29) || seqlen_add > 1 << 30) return py::none();
   const float *ks, *vs, *sink_ptr, *alibi_ptr;
   if (!head_vector(sinks, hq, device, sink_ptr) || !head_vector(alibi_slopes, hq, device, alibi_ptr))
@@ -548,7 +550,8 @@ py::object decode_tokens(const at::Tensor &q, const at::Tensor &k_cache, const a
         fp8                  ? MXFA_DTYPE_FP8_E4M3
         : dt == at::kBFloat16 ? MXFA_DTYPE_BF16
                               : MXFA_DTYPE_F16,
-        ks, vs, ns, stream);
+        ks, vs, ns, advance && t + n == ql ? cache_seqlens.data_ptr<int32_t>() : nullptr,
+        (int)advance, stream);
     if (t == 0 && (rc == MXFA_EUNSUPPORTED || rc == MXFA_EINVAL))
       return py::none();  // nothing launched
     if (rc != MXFA_OK)
@@ -672,7 +675,7 @@ PYBIND11_MODULE(_mxfa_torch, m) {
         py::arg("block_table"), py::arg("cache_seqlens"), py::arg("scale"), py::arg("out"),
         py::arg("num_splits"), py::arg("seqlen_add"), py::arg("causal"), py::arg("window_left"),
         py::arg("softcap"), py::arg("k_scale"), py::arg("v_scale"), py::arg("sinks"),
-        py::arg("alibi_slopes"));
+        py::arg("alibi_slopes"), py::arg("advance") = 0);
   m.def("reshape_and_cache", &reshape_and_cache, py::arg("key"), py::arg("value"),
         py::arg("key_cache"), py::arg("value_cache"), py::arg("slot_mapping"),
         py::arg("k_scale") = py::none(), py::arg("v_scale") = py::none());

@@ -133,6 +133,12 @@ def route_kvcache(q, k_cache, v_cache, k, v, cache_seqlens, block_table, scale,
         new = 0 if k is None else k.shape[1]
         if new:
             native.append_kv(k, v, kc, vc, table, cache_seqlens)
+            op = native.torch_op() if native.USE_TORCH_OP else None
+            if op is not None:  # the decode's last launch moves the lengths on
+                result = op.decode_tokens(q, kc, vc, table, cache_seqlens, scale, out, None, new,
+                                          bool(causal), -1, 0.0, None, None, None, None, new)
+                if result is not None:
+                    return result if out is None else out
         result = native.paged_decode_split(q, kc, vc, table, cache_seqlens, scale,
                                            seqlen_add=new, causal=causal, out=out)
         if new:

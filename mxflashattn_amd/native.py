@@ -151,7 +151,8 @@ _SIGNATURES = {
 # Entry points for this package only (csrc/mxfa_package.h), not part of the C ABI.
 _PACKAGE_SIGNATURES = {
     "mxfa_package_launch_columns": (_i, [_i, _i, _i, _i]),
-    "mxfa_package_decode_tokens_launch": _SIGNATURES["mxfa_split_decode_multi_launch"],
+    "mxfa_package_decode_tokens_launch": (
+        _i, [*_SIGNATURES["mxfa_split_decode_multi_launch"][1][:-1], _p, _i, _p]),
 }
 
 _load_lock = threading.Lock()
@@ -573,7 +574,7 @@ def _launch_multi(q, k_cache, v_cache, block_table, cache_seqlens, out, workspac
         ws_bytes, float(softmax_scale), batch, hq, hkv, hd, ps, block_table.shape[1], pages,
         DTYPE_CODES[q.dtype], DTYPE_FP8_E4M3 if fp8 else DTYPE_CODES[q.dtype],
         _scale_ptr(k_scale, q.device, "k_scale") if fp8 else 0,
-        _scale_ptr(v_scale, q.device, "v_scale") if fp8 else 0, num_splits, stream)
+        _scale_ptr(v_scale, q.device, "v_scale") if fp8 else 0, num_splits, 0, 0, stream)
     _check(rc, "mxfa_split_decode_multi_launch")
 
 
