@@ -42,30 +42,47 @@ struct AppendParams {
   int num_pages;
 };
 
-template <bool kTable>
+// Small appends are bound by latency: the index arithmetic, then the length or
+// slot, then the page id, then the row. All of the arithmetic ran in 64 bits,
+// whose divisions are long software sequences ahead of every load; I = uint32_t
+// (appends of fewer than 2^31 fragments) divides in 32 bits, and positions and
+// slots do too where they fit. Measured on MI355X (us a call): the fp8 append and
+// decode of one layer, 128 sequences of 8 kv heads, HD 128, 77.43 -> 76.97; 8192
+// rows of 8 heads, HD 128, bf16, 11.33 -> 11.20 (6.0 TB/s read and written).
+__device__ __forceinline__ void page_of(int64_t pos, int ps, int64_t &page, int64_t &off) {
+  if (pos <= 0x7fffffff) {
+    const uint32_t q = (uint32_t)pos / (uint32_t)ps;
+    page = q;
+    off = (uint32_t)pos - q * (uint32_t)ps;
+  } else {
+    page = pos / ps;
+    off = pos % ps;
+  }
+}
+
+template <bool kTable, typename I>
 __global__ __launch_bounds__(256) void kv_append_kernel(AppendParams p) {
-  const int64_t total = (int64_t)p.rows * p.hkv * p.frags;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int f = (int)(i % p.frags);
-    const int64_t rh = i / p.frags;
-    const int h = (int)(rh % p.hkv);
-    const int r = (int)(rh / p.hkv);
+  const I total = (I)p.rows * (I)p.hkv * (I)p.frags;
+  const I stride = (I)gridDim.x * 256;
+  for (I i = (I)blockIdx.x * 256 + threadIdx.x; i < total; i += stride) {
+    const I rh = i / (I)p.frags;
+    const int f = (int)(i - rh * (I)p.frags);
+    const int r = (int)(rh / (I)p.hkv);
+    const int h = (int)(rh - (I)r * (I)p.hkv);
     int64_t page, off, src;
     if (kTable) {
-      const int b = r / p.new_tokens, t = r % p.new_tokens;
+      const int b = r / p.new_tokens, t = r - b * p.new_tokens;
       const int64_t pos = (int64_t)p.seqlens[b] + t;
       if (pos < 0) continue;
-      const int64_t pidx = pos / p.ps;
+      int64_t pidx;
+      page_of(pos, p.ps, pidx, off);
       if (pidx >= p.btw) continue;
       page = p.bt[(int64_t)b * p.bt_stride + pidx];
-      off = pos % p.ps;
       src = (int64_t)b * p.s_b + (int64_t)t * p.s_t;
     } else {
       const int64_t slot = p.slots[r];
       if (slot < 0) continue;
-      page = slot / p.ps;
-      off = slot % p.ps;
+      page_of(slot, p.ps, page, off);
       src = (int64_t)r * p.s_t;
     }
     if (page < 0 || page >= p.num_pages) continue;
@@ -116,20 +133,21 @@ __device__ __forceinline__ uint2 quantize8(const uint4 w, float s) {
   return make_uint2(out[0], out[1]);
 }
 
-template <typename T>
+template <typename T, typename I>
 __global__ __launch_bounds__(256) void kv_quant_append_kernel(QuantAppendParams p) {
   const float ks = p.k_scale ? p.k_scale[0] : 1.f;
   const float vs = p.v_scale ? p.v_scale[0] : 1.f;
-  const int64_t total = (int64_t)p.rows * p.hkv * p.frags;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int f = (int)(i % p.frags);
-    const int64_t rh = i / p.frags;
-    const int h = (int)(rh % p.hkv);
-    const int r = (int)(rh / p.hkv);
+  const I total = (I)p.rows * (I)p.hkv * (I)p.frags;
+  const I stride = (I)gridDim.x * 256;
+  for (I i = (I)blockIdx.x * 256 + threadIdx.x; i < total; i += stride) {
+    const I rh = i / (I)p.frags;
+    const int f = (int)(i - rh * (I)p.frags);
+    const int r = (int)(rh / (I)p.hkv);
+    const int h = (int)(rh - (I)r * (I)p.hkv);
     const int64_t slot = p.slots[r];
     if (slot < 0) continue;
-    const int64_t page = slot / p.ps, off = slot % p.ps;
+    int64_t page, off;
+    page_of(slot, p.ps, page, off);
     if (page >= p.num_pages) continue;
     const int64_t src = (int64_t)r * p.s_t + (int64_t)h * p.s_h + f * 8;
     const int64_t dst = page * p.c_sp + off * p.c_st + (int64_t)h * p.c_sh + f * 8;
@@ -140,6 +158,10 @@ __global__ __launch_bounds__(256) void kv_quant_append_kernel(QuantAppendParams 
   }
 }
 
+// A grid-stride step past the last fragment must not wrap either: at most 2^24
+// threads step at once.
+constexpr int64_t kIndex32Max = ((int64_t)1 << 31) - ((int64_t)1 << 24);
+
 static bool al16(const void *ptr) { return ((uintptr_t)ptr & 15u) == 0; }
 
 template <bool kTable>
@@ -148,7 +170,12 @@ static int launch_append(const AppendParams &p, hipStream_t st) {
   if (total == 0) return MXFA_OK;
   int64_t blocks = (total + 255) / 256;
   if (blocks > 65536) blocks = 65536;
-  hipLaunchKernelGGL((kv_append_kernel<kTable>), dim3((unsigned)blocks), dim3(256), 0, st, p);
+  if (total <= kIndex32Max)
+    hipLaunchKernelGGL((kv_append_kernel<kTable, uint32_t>), dim3((unsigned)blocks), dim3(256), 0,
+                       st, p);
+  else
+    hipLaunchKernelGGL((kv_append_kernel<kTable, int64_t>), dim3((unsigned)blocks), dim3(256), 0,
+                       st, p);
   return hipGetLastError() == hipSuccess ? MXFA_OK : MXFA_ELAUNCH;
 }
 
@@ -247,12 +274,16 @@ int mxfa_reshape_and_cache_fp8_launch(const void *key, const void *value,
   int64_t blocks = (total + 255) / 256;
   if (blocks > 65536) blocks = 65536;
   hipStream_t st = (hipStream_t)stream;
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, st, p);
+  };
+  const bool i32 = total <= kIndex32Max;
   if (dtype == MXFA_DTYPE_BF16)
-    hipLaunchKernelGGL((kv_quant_append_kernel<BF16>), dim3((unsigned)blocks), dim3(256), 0, st,
-                       p);
+    i32 ? launch(kv_quant_append_kernel<BF16, uint32_t>)
+        : launch(kv_quant_append_kernel<BF16, int64_t>);
   else
-    hipLaunchKernelGGL((kv_quant_append_kernel<F16>), dim3((unsigned)blocks), dim3(256), 0, st,
-                       p);
+    i32 ? launch(kv_quant_append_kernel<F16, uint32_t>)
+        : launch(kv_quant_append_kernel<F16, int64_t>);
   return hipGetLastError() == hipSuccess ? MXFA_OK : MXFA_ELAUNCH;
 }
 
