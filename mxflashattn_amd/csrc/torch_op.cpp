@@ -676,9 +676,19 @@ PYBIND11_MODULE(_mxfa_torch, m) {
         py::arg("num_splits"), py::arg("seqlen_add"), py::arg("causal"), py::arg("window_left"),
         py::arg("softcap"), py::arg("k_scale"), py::arg("v_scale"), py::arg("sinks"),
         py::arg("alibi_slopes"), py::arg("advance") = 0);
-  m.def("reshape_and_cache", &reshape_and_cache, py::arg("key"), py::arg("value"),
+  // The call without scales by itself: two optional arguments cost a small
+  // append 0.1 us of its 4.1 us.
+  m.def("reshape_and_cache",
+        [](const at::Tensor &key, const at::Tensor &value, const at::Tensor &key_cache,
+           const at::Tensor &value_cache, const at::Tensor &slot_mapping) {
+          return reshape_and_cache(key, value, key_cache, value_cache, slot_mapping, c10::nullopt,
+                                   c10::nullopt);
+        },
+        py::arg("key"), py::arg("value"), py::arg("key_cache"), py::arg("value_cache"),
+        py::arg("slot_mapping"));
+  m.def("reshape_and_cache_scaled", &reshape_and_cache, py::arg("key"), py::arg("value"),
         py::arg("key_cache"), py::arg("value_cache"), py::arg("slot_mapping"),
-        py::arg("k_scale") = py::none(), py::arg("v_scale") = py::none());
+        py::arg("k_scale"), py::arg("v_scale"));
   m.def("append_kv", &append_kv, py::arg("k"), py::arg("v"), py::arg("k_cache"),
         py::arg("v_cache"), py::arg("block_table"), py::arg("cache_seqlens"));
   m.def("abi_version", &mxfa_abi_version);

@@ -37,7 +37,8 @@ _ACCEL = {"cuda"}
 
 def _query_length_reason(q: torch.Tensor, kv_heads: int, causal: bool) -> str | None:
     """q is [B, QL, HQ, D]: QL query tokens x GQ heads fill the kernel's columns,
-    or, for a causal query, up to four launches of them (token chunks)."""
+    or, for a causal query, up to four times as many (column groups, or token
+    chunks)."""
     ql, gq = q.shape[1], q.shape[-2] // kv_heads
     limit = native.CHUNKED_COLUMNS if causal else native.KERNEL_COLUMNS
     if ql < 1 or ql * gq > limit:

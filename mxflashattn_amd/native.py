@@ -909,7 +909,7 @@ def reshape_and_cache(
             if k_scale is None and v_scale is None:
                 if op.reshape_and_cache(key, value, key_cache, value_cache, slot_mapping):
                     return
-            elif _op_scales(k_scale, v_scale) and op.reshape_and_cache(
+            elif _op_scales(k_scale, v_scale) and op.reshape_and_cache_scaled(
                     key, value, key_cache, value_cache, slot_mapping, k_scale, v_scale):
                 return
     if key.dim() != 3 or value.shape != key.shape:
