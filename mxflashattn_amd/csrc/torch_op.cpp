@@ -342,18 +342,28 @@ py::object contiguous_decode(const at::Tensor &q, const at::Tensor &k, const at:
     out = at::empty(q.sizes(), q.options());
     strides(out, os);
   }
-  // The heuristic as for pages of 16 tokens, asked for the columns of one
-  // launch; past 16 columns it is asked again unless it picked the
-  // per-sequence kernel.
-  const int cus = num_cus(device.index()), width = (int)((max_len + 15) / 16);
+  // The heuristic as for the pages of the same bytes (decode.py): one-token
+  // pages for packed keys, for a dense cache the largest power of two dividing
+  // its length, up to 256. Asked with pages of 16 it gave short sequences to the
+  // per-sequence kernel, whose waves hold several tiles against one reference
+  // maximum: the largest weight of a tile is then no longer exactly 1 before P
+  // is rounded, and the error against 64 bits grew by up to 19 % (fp16, HD 64,
+  // 8q/2kv, sequences of 500-767 keys: 2.45e-4 -> 2.87e-4; bf16 1.96e-3 ->
+  // 2.30e-3). Splitting them costs 1-4 us a call (5 packed sequences and up:
+  // 33 -> 34.5 us; a dense call 15.2 -> 19.1 us, with the second launch).
+  // Asked for the columns of one launch; past 16 columns it is asked again
+  // unless it picked the per-sequence kernel.
+  const int64_t rows = packed ? 1 : k.size(1);
+  const int ps = (int)std::min<int64_t>(rows & -rows, 256);
+  const int cus = num_cus(device.index()), width = (int)((max_len + ps - 1) / ps);
   const int64_t gq = hq / hkv;
   const int64_t first_ask = std::min<int64_t>(ql, std::max<int64_t>(1, 16 / gq));
   int ns = 0;
-  if (mxfa_split_heuristic((int)batch, (int)(hq * first_ask), (int)hkv, (int)hd, 16, width, cus,
+  if (mxfa_split_heuristic((int)batch, (int)(hq * first_ask), (int)hkv, (int)hd, ps, width, cus,
                            &ns) != MXFA_OK)
     return py::none();
   if (first_ask < ql && ns != MXFA_SPLITS_PER_SEQUENCE &&
-      mxfa_split_heuristic((int)batch, (int)(hkv * 17), (int)hkv, (int)hd, 16, width, cus, &ns) !=
+      mxfa_split_heuristic((int)batch, (int)(hkv * 17), (int)hkv, (int)hd, ps, width, cus, &ns) !=
           MXFA_OK)
     return py::none();
   size_t ws_bytes = 0;

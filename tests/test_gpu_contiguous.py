@@ -59,16 +59,29 @@ def test_packed_rows(device, monkeypatch, hd, gq, dtype, wide):
     assert torch.equal(out, paged)  # the same tiles, ranges and arithmetic
 
 
-def test_short_packed_sequences_take_the_per_sequence_kernel(device):
+@pytest.mark.parametrize("hd", [64, 128])
+def test_short_packed_sequences_are_split_as_their_pages(device, monkeypatch, hd):
+    # Sequences short enough for the per-sequence kernel, which rounds more
+    # weights against one reference maximum: one-token pages never took it.
     lens = [1, 16, 200, 255, 31]
-    k, v = (randn(sum(lens), 2, 64, dtype=torch.float16, seed=s) for s in (1, 2))
-    q = randn(5, 8, 64, dtype=torch.float16, seed=3)
+    k, v = (randn(sum(lens), 2, hd, dtype=torch.float16, seed=s) for s in (1, 2))
+    q = randn(5, 8, hd, dtype=torch.float16, seed=3)
     cu_q, cu_k = torch.arange(6), torch.tensor([0, *torch.tensor(lens).cumsum(0).tolist()])
     ref = reference_port.attention_varlen(q.float(), k.float(), v.float(), cu_q.tolist(),
-                                          cu_k.tolist(), softmax_scale=0.125)
-    out = mx.flash_attn_varlen_func(q.to(device), k.to(device), v.to(device), cu_q.to(device),
-                                    cu_k.to(device), 1, 255)
+                                          cu_k.tolist(), softmax_scale=hd ** -0.5)
+    out, paged = both_routes(monkeypatch, lambda: mx.flash_attn_varlen_func(
+        q.to(device), k.to(device), v.to(device), cu_q.to(device), cu_k.to(device), 1, 255))
     close(out, ref, torch.float16)
+    assert torch.equal(out, paged)
+
+
+@pytest.mark.parametrize("seq", [33, 129, 250, 383])  # pages of 1 or 2 tokens
+@pytest.mark.parametrize("hd", [64, 128])
+def test_short_odd_dense_keys_are_split_as_their_pages(device, monkeypatch, seq, hd):
+    k, v = (randn(4, seq, 2, hd, dtype=torch.bfloat16, seed=s).to(device) for s in (1, 2))
+    q = randn(4, 1, 8, hd, dtype=torch.bfloat16, seed=3).to(device)
+    out, paged = both_routes(monkeypatch, lambda: mx.flash_attn_func(q, k, v, causal=True))
+    assert torch.equal(out, paged)
 
 
 @pytest.mark.parametrize("seq", [1, 15, 47, 96, 1025, 2048])
