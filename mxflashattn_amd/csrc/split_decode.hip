@@ -142,6 +142,7 @@ struct SplitArgs {
   int advance_by;
   bool contiguous;     // a sequence's keys are consecutive rows: one page per sequence (ps 1,
                        // btw = the longest sequence, bt = its first row or page, bt_stride 1)
+  int same_pages;      // contiguous: page size of the pages that hold the same bytes
 };
 
 struct WsLayout {
@@ -289,6 +290,9 @@ static int launch_partial(const SplitArgs &a, hipStream_t st) {
   // capacity (the lengths are on the device).
   const int64_t cap_tiles = ((int64_t)a.btw * a.ps + kTile - 1) / kTile;
   g.short_ranges = (int64_t)a.batch * cap_tiles <= (int64_t)kShortRangeTiles * a.num_splits;
+  // Keys in consecutive rows give the bits of the pages that hold them: of
+  // pages shorter than a tile QK is on the matrix cores (0.5 % of a call).
+  g.mfma_qk = a.contiguous && a.same_pages < kTile;
   const DecodeParams p = make_params(a, g);
   // The tile scan: inside each wave, one or four sequences per lane, or
   // through LDS; four per lane is built for plain calls only.
@@ -420,6 +424,7 @@ static SplitArgs split_args(const void *q, int64_t q_stride_b, int64_t q_stride_
   a.advance = nullptr;
   a.advance_by = 0;
   a.contiguous = false;
+  a.same_pages = 0;
   return a;
 }
 
@@ -835,10 +840,10 @@ int mxfa_package_contiguous_decode_launch(
     int causal, const void *k, const void *v, int64_t first_stride, int64_t token_stride,
     int64_t head_stride, int64_t num_firsts, int max_len, const void *cu_seqlens_q,
     int cu_q_is_int64, const void *cu_seqlens_k, int cu_k_is_int64, int num_seqs,
-    int64_t *host_offsets, void *offsets_event, const int32_t *seqlens, int seqlen_add, void *out, int64_t out_stride_b,
-    int64_t out_stride_t, int64_t out_stride_h, void *workspace, size_t workspace_bytes,
-    float scale, int batch, int q_heads, int kv_heads, int head_dim, int dtype, int num_splits,
-    void *stream) {
+    int64_t *host_offsets, void *offsets_event, const int32_t *seqlens, int seqlen_add,
+    void *out, int64_t out_stride_b, int64_t out_stride_t, int64_t out_stride_h, void *workspace,
+    size_t workspace_bytes, float scale, int batch, int q_heads, int kv_heads, int head_dim,
+    int page_size, int dtype, int num_splits, void *stream) {
   size_t need = 0;
   int rc = mxfa_package_contiguous_workspace_size(batch, q_heads, kv_heads, q_len, head_dim,
                                                   num_splits, &need);
@@ -858,6 +863,7 @@ int mxfa_package_contiguous_decode_launch(
                            q_heads, kv_heads, head_dim, 1, max_len, (int)num_firsts, dtype,
                            num_splits);
   a.contiguous = true;
+  a.same_pages = page_size;
   a.q_st = q_stride_t;
   a.o_st = out_stride_t;
   a.causal = causal;

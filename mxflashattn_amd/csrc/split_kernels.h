@@ -148,6 +148,7 @@ struct DecodeParams {
 struct Grid {
   int waves, heads_per_wg, subs, gx, gy;
   bool short_ranges = false;  // host's bound on tiles per range <= kShortRangeTiles
+  bool mfma_qk = false;       // QK on the matrix cores whatever the columns (valu_qk_columns)
 };
 
 struct CombineParams {
@@ -1877,9 +1878,7 @@ static int launch_partial_hr(const DecodeParams &p, const Grid &g, hipStream_t s
   switch (head_rows(cols)) {
     case 1:
       if constexpr (!kF8 && HD >= 128) {
-        // Keys in consecutive rows take QK on the matrix cores: the same bits
-        // as the same keys read as one-token pages (about 0.5 % of a call).
-        if (p.ps_log2 >= 4 && p.ps_log2 != kContiguousLog2) {
+        if (p.ps_log2 >= 4 && !g.mfma_qk) {
           switch (valu_qk_columns(cols, HD)) {
             case 1: return launch_partial_t<HD, 1, T, kF8, kWaveScan, 1>(p, g, st);
             case 2: return launch_partial_t<HD, 1, T, kF8, kWaveScan, 2>(p, g, st);

@@ -386,9 +386,9 @@ py::object contiguous_decode(const at::Tensor &q, const at::Tensor &k, const at:
   const int rc = mxfa_package_contiguous_decode_launch(
       q.data_ptr(), qs[0], qs[1], qs[2], (int)ql, causal, k.data_ptr(), v.data_ptr(), k.stride(0),
       token_stride, k.stride(-2), firsts, (int)max_len, cu_q, cu_q64, cu_k, cu_k64, (int)num_seqs,
-      host_offsets, offsets ? offsets->event() : nullptr, seqlens, 0, out.data_ptr(), os[0], os[1], os[2], ws.data_ptr(), ws_bytes, (float)scale,
-      (int)batch, (int)hq, (int)hkv, (int)hd, dt == at::kBFloat16 ? MXFA_DTYPE_BF16 : MXFA_DTYPE_F16,
-      ns, stream);
+      host_offsets, offsets ? offsets->event() : nullptr, seqlens, 0, out.data_ptr(), os[0],
+      os[1], os[2], ws.data_ptr(), ws_bytes, (float)scale, (int)batch, (int)hq, (int)hkv, (int)hd,
+      ps, dt == at::kBFloat16 ? MXFA_DTYPE_BF16 : MXFA_DTYPE_F16, ns, stream);
   if (rc == MXFA_EUNSUPPORTED || rc == MXFA_EINVAL) return py::none();  // nothing launched
   if (offsets) {
     if (rc != MXFA_OK) (void)hipStreamSynchronize((hipStream_t)stream);  // no event to wait for
