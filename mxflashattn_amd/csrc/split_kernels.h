@@ -1127,6 +1127,18 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
     });
   };
 
+  // Several groups where 16 columns run in twice the ranges (more than four kv
+  // heads, rows of up to 128 bytes: waves_for): the second tile of a piece moves
+  // the reference to its own maximum too, up or down, so that of every two tiles
+  // as many weights are exactly 1 before P is rounded as in two pieces of half
+  // the length. Error against 64 bits (bf16, HD 64, 16q/8kv, 12 tokens, 500-1000
+  // keys, B 4): 16 columns a launch 1.951e-3, one reference a piece 2.075e-3, two
+  // 1.951e-3; for 0-6 % of a call (B 32, 12 tokens of 32q/8kv, 1k-8k keys 97.7 ->
+  // 102.1 us; twice the ranges instead cost 5-35 %: 113.1 us).
+  constexpr bool kTwoExact = kGroups > 1 && HD * (kF8 ? 1 : 2) <= 128;
+  const float second_move = kTwoExact && p.hkv > 4 ? -INFINITY : kRescaleLog2;
+  bool after_first = false;  // the last tile was its piece's first
+
   uint32_t probe = 0;
   auto compute = [&](Set &s) {
     const Tile &d = s.d;
@@ -1231,6 +1243,9 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
         }
       }
     }
+    // The reference moves when a score passes it by more than this.
+    const float move = kTwoExact && after_first ? second_move : kRescaleLog2;
+    after_first = (d.flags & kFirst) != 0;
     uint2 a[kGroups];  // P of each group, packed pairs of the element type
     static_for<kGroups>([&](auto gc) {
       constexpr int g = decltype(gc)::value;
@@ -1258,7 +1273,7 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
         bool valid = (16 * g + col < nc) & (r < d.rem - c_hide[g]);
         if constexpr (kExtras) valid &= r >= d.rem - c_reach[g];
         x[i] = valid ? x[i] : -INFINITY;
-        need |= x[i] > m[g] + kRescaleLog2;
+        need |= x[i] > m[g] + move;
       }
 #ifdef MXFA_WAVE_STAMPS
       if (stamp_data) {
@@ -1270,7 +1285,8 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
         // Rare, wave-uniform: move the reference of each head to the wave's
         // tile maximum when it passed the reference by more than kRescaleLog2.
         const float mt = rows_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
-        const float mn = mt > m[g] + kRescaleLog2 ? mt : m[g];
+        const float to = kTwoExact ? fmaxf(mt, m[g] - kRescaleLog2) : mt;
+        const float mn = mt > m[g] + move ? to : m[g];
         const float f = (mn == m[g]) ? 1.f : fast_exp2(m[g] - mn);  // m = -inf: f = 0
         dsum[g] *= f;
         static_for<4>([&](auto ic) {
@@ -1916,13 +1932,14 @@ int launch_partial_hd(const DecodeParams &p, const Grid &g, int dtype, bool fp8,
 // sinks or ALiBi; two with fp8 caches (a third register set and the widened
 // operands); one at head dim 256.
 // Measured on MI355X against launches of 16 columns that each read the keys
-// again (graph replays, B 32, 8 kv heads, GQ 4, bf16, L ~ U[2048, 4096], us per
-// call): head dim 128, 5 tokens 141.4 -> 80.4, 8 tokens 154.2 -> 85.0, 12 tokens
-// 228.8 -> 94.8, 16 tokens (two launches instead of four) 296.5 -> 167.2; head
-// dim 64, 8 tokens 90.7 -> 50.8, 16 tokens 174.5 -> 75.4. One pass over the
-// keys is bound by HBM up to 32 columns at head dim 128 (85 us against 79 for
-// one token); past that, and at head dim 64, each group's softmax and matrix
-// instructions show, since one wave per SIMD has nothing to hide them behind.
+// again (calls in a row, B 32, 8 kv heads, GQ 4, bf16, L ~ U[2048, 4096], us per
+// call): head dim 128, 5 tokens 133.8 -> 72.9, 8 tokens 138.1 -> 78.7, 12 tokens
+// 207.8 -> 87.8, 16 tokens (two launches instead of four) 275.7 -> 155.3; head
+// dim 64, 8 tokens 83.3 -> 47.0, 12 tokens 125.2 -> 72.8, 16 tokens 167.2 ->
+// 75.9. One pass over the keys is bound by HBM up to 32 columns at head dim 128
+// (79 us for 8 tokens, 73 for 5); past that, and at head dim 64, each group's
+// softmax and matrix instructions show, since one wave per SIMD has nothing to
+// hide them behind.
 template <int HD, bool kF8, bool kExtras>
 constexpr int kMostGroups = HD > 128 ? 1 : kF8 ? 2 : HD == 64 ? 4 : kExtras ? 2 : 3;
 
