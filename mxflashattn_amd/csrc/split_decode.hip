@@ -562,6 +562,9 @@ static int run_tokens(SplitArgs a, int64_t q_stride_t, int q_len, int causal, in
 // sequences without a row are left out. Rows no sequence names get length 0,
 // and start and length are held to the total_rows rows that exist, so offsets
 // that do not describe the keys give wrong numbers, never a read outside them.
+// For the same reason a row that several sequences name (offsets that have not
+// been checked yet) takes start and length from one of them: one thread writes
+// both, from the sequence left in LDS.
 constexpr int kRowsThreads = 1024;
 struct RowsParams {
   const void *cu_q;
@@ -580,28 +583,40 @@ __global__ __launch_bounds__(kRowsThreads) void contiguous_rows_kernel(RowsParam
   const auto at = [](const void *cu, int wide, int i) -> int64_t {
     return wide ? static_cast<const int64_t *>(cu)[i] : static_cast<const int32_t *>(cu)[i];
   };
-  for (int r = threadIdx.x; r < p.batch; r += kRowsThreads) {
-    p.first[r] = p.cu_k ? 0 : r;
-    p.len[r] = p.cu_k ? 0 : p.max_len;
+  if (!p.cu_k) {
+    for (int r = threadIdx.x; r < p.batch; r += kRowsThreads) {
+      p.first[r] = r;
+      p.len[r] = p.max_len;
+    }
+    return;
   }
-  if (!p.cu_k) return;
+  extern __shared__ int32_t s_seq[];  // the sequence of each query row, -1: none
+  for (int r = threadIdx.x; r < p.batch; r += kRowsThreads) s_seq[r] = -1;
+  __syncthreads();
+  for (int i = threadIdx.x; i < p.num_seqs; i += kRowsThreads) {
+    const int64_t r = at(p.cu_q, p.q64, i), r1 = at(p.cu_q, p.q64, i + 1);
+    if (r1 > r && r >= 0 && r < p.batch) s_seq[r] = i;
+  }
   __syncthreads();
   // The caller's copy of the offsets (it checks them while the decode runs):
-  // num_seqs + 1 of cu_q, then of cu_k.
+  // num_seqs + 1 of cu_q, then of cu_k. Past the last barrier, which would wait
+  // for these stores.
   if (p.host_offsets) {
     for (int i = threadIdx.x; i <= p.num_seqs; i += kRowsThreads) {
       p.host_offsets[i] = at(p.cu_q, p.q64, i);
       p.host_offsets[p.num_seqs + 1 + i] = at(p.cu_k, p.k64, i);
     }
   }
-  for (int i = threadIdx.x; i < p.num_seqs; i += kRowsThreads) {
-    const int64_t r = at(p.cu_q, p.q64, i), r1 = at(p.cu_q, p.q64, i + 1);
-    if (r1 <= r || r < 0 || r >= p.batch) continue;
-    const int64_t k0 = at(p.cu_k, p.k64, i), k1 = at(p.cu_k, p.k64, i + 1);
-    const int64_t first = k0 < 0 ? 0 : k0 > p.total_rows ? p.total_rows : k0;
-    int64_t n = k1 - first;
-    n = n > p.total_rows - first ? p.total_rows - first : n;
-    n = n > p.max_len ? p.max_len : n;
+  for (int r = threadIdx.x; r < p.batch; r += kRowsThreads) {
+    const int i = s_seq[r];
+    int64_t first = 0, n = 0;
+    if (i >= 0) {
+      const int64_t k0 = at(p.cu_k, p.k64, i), k1 = at(p.cu_k, p.k64, i + 1);
+      first = k0 < 0 ? 0 : k0 > p.total_rows ? p.total_rows : k0;
+      n = k1 - first;
+      n = n > p.total_rows - first ? p.total_rows - first : n;
+      n = n > p.max_len ? p.max_len : n;
+    }
     p.first[r] = (int32_t)first;
     p.len[r] = n > 0 ? (int32_t)n : 0;
   }
@@ -884,7 +899,8 @@ int mxfa_package_contiguous_decode_launch(
       RowsParams r{cu_seqlens_q, cu_seqlens_k, cu_q_is_int64, cu_k_is_int64, num_seqs,
                    num_firsts,   max_len,      batch,         first,         first + batch,
                    host_offsets};
-      hipLaunchKernelGGL(contiguous_rows_kernel, dim3(1), dim3(kRowsThreads), 0, st, r);
+      const size_t lds = cu_seqlens_k ? (size_t)batch * sizeof(int32_t) : 0;
+      hipLaunchKernelGGL(contiguous_rows_kernel, dim3(1), dim3(kRowsThreads), lds, st, r);
       if (hipGetLastError() != hipSuccess) return MXFA_ELAUNCH;
       if (offsets_event && hipEventRecord((hipEvent_t)offsets_event, st) != hipSuccess)
         return MXFA_ELAUNCH;

@@ -135,6 +135,27 @@ def test_offsets_that_name_no_keys_read_nothing_outside(device):
         close(out[b], want, torch.float16)
 
 
+def test_a_row_that_several_sequences_name_takes_one_of_them(device):
+    # Offsets the API refuses once it has read them; the kernels are out by then.
+    # 200 sequences, every other one of query row 0: the first of all keys, the
+    # last (in another wave) of the last key. A first row of one with the length
+    # of the other would pass the keys' end.
+    op = native.torch_op()
+    k, v = (randn(100, 2, 64, dtype=torch.float16, seed=s).to(device) for s in (5, 6))
+    q = randn(1, 4, 64, dtype=torch.float16, seed=7).to(device)
+    cu_q = torch.arange(201, dtype=torch.int32, device=device) % 2
+    cu_k = torch.tensor([0, 100] + [50, 60] * 98 + [99, 100, 100], dtype=torch.int32,
+                        device=device)
+    out = op.contiguous_decode(q, k, v, 0.125, False, 100, cu_q, cu_k)
+    want = [reference_port.attention_single(q.float().cpu(), k[a:e].float().cpu(),
+                                            v[a:e].float().cpu(), softmax_scale=0.125)
+            for a, e in ((0, 100), (50, 60), (99, 100))]
+    errs = [(out.float().cpu() - w).abs().max().item() for w in want]
+    assert min(errs) <= TOL[torch.float16], errs
+    with pytest.raises(ValueError, match="cu_seqlens_q must start at zero"):
+        mx.flash_attn_varlen_func(q, k, v, cu_q, cu_k, 1, 100)
+
+
 def test_packed_offsets_are_checked_after_the_launch(device):
     """Offsets the API rejects raise the same errors as before the kernels
     went out first, leave the next call right, and name no row outside."""
