@@ -622,14 +622,6 @@ __global__ __launch_bounds__(kRowsThreads) void contiguous_rows_kernel(RowsParam
   }
 }
 
-// Workspace of a contiguous call: the split workspace of `rows` = q heads x
-// query tokens of one launch, then first rows and lengths.
-static size_t contiguous_ws(int batch, int rows, int hd, int ns, size_t *tail) {
-  const size_t split = ns > 0 ? ws_layout(batch, rows, hd, ns).bytes : 0;
-  *tail = (split + 15) & ~(size_t)15;
-  return *tail + (size_t)batch * 2 * sizeof(int32_t);
-}
-
 // Query tokens of one launch of a contiguous call: all of them, or for a
 // causal query of more columns as many as fit (about equal shares where a
 // launch takes several column groups).
@@ -845,8 +837,7 @@ int mxfa_package_contiguous_workspace_size(int batch, int q_heads, int kv_heads,
       (num_splits <= 0 && num_splits != MXFA_SPLITS_PER_SEQUENCE))
     return MXFA_EINVAL;
   const int tokens = contiguous_tokens(q_len, q_heads / kv_heads, head_dim, num_splits);
-  size_t tail;
-  *bytes = contiguous_ws(batch, q_heads * tokens, head_dim, num_splits, &tail);
+  *bytes = num_splits > 0 ? ws_layout(batch, q_heads * tokens, head_dim, num_splits).bytes : 0;
   return MXFA_OK;
 }
 
@@ -855,28 +846,26 @@ int mxfa_package_contiguous_decode_launch(
     int causal, const void *k, const void *v, int64_t first_stride, int64_t token_stride,
     int64_t head_stride, int64_t num_firsts, int max_len, const void *cu_seqlens_q,
     int cu_q_is_int64, const void *cu_seqlens_k, int cu_k_is_int64, int num_seqs,
-    int64_t *host_offsets, void *offsets_event, const int32_t *seqlens, int seqlen_add,
-    void *out, int64_t out_stride_b, int64_t out_stride_t, int64_t out_stride_h, void *workspace,
-    size_t workspace_bytes, float scale, int batch, int q_heads, int kv_heads, int head_dim,
-    int page_size, int dtype, int num_splits, void *stream) {
+    int32_t *rows, int64_t *host_offsets, void *offsets_event, const int32_t *seqlens,
+    int seqlen_add, void *out, int64_t out_stride_b, int64_t out_stride_t, int64_t out_stride_h,
+    void *workspace, size_t workspace_bytes, float scale, int batch, int q_heads, int kv_heads,
+    int head_dim, int page_size, int dtype, int num_splits, void *stream) {
   size_t need = 0;
   int rc = mxfa_package_contiguous_workspace_size(batch, q_heads, kv_heads, q_len, head_dim,
                                                   num_splits, &need);
   if (rc != MXFA_OK) return rc;
-  if (!workspace || !aligned16(workspace) || workspace_bytes < need) return MXFA_EWORKSPACE;
+  if (workspace_bytes < need) return MXFA_EWORKSPACE;
+  if (!rows || ((uintptr_t)rows & 3u)) return MXFA_EINVAL;
   if (num_firsts <= 0 || num_firsts > INT32_MAX || max_len <= 0) return MXFA_EINVAL;
   if (cu_seqlens_k ? (!cu_seqlens_q || num_seqs < batch || seqlens) : num_firsts < batch)
     return MXFA_EINVAL;
   const int tokens = contiguous_tokens(q_len, q_heads / kv_heads, head_dim, num_splits);
   if (tokens < q_len && !causal) return MXFA_EUNSUPPORTED;
-  size_t tail = 0;
-  contiguous_ws(batch, q_heads * tokens, head_dim, num_splits, &tail);
-  int32_t *first = (int32_t *)((char *)workspace + tail);
   SplitArgs a = split_args(q, q_stride_b, q_stride_h, k, v, first_stride, token_stride,
-                           head_stride, first, 1, seqlens ? seqlens : first + batch, seqlen_add,
-                           out, out_stride_b, out_stride_h, workspace, tail, scale, batch,
-                           q_heads, kv_heads, head_dim, 1, max_len, (int)num_firsts, dtype,
-                           num_splits);
+                           head_stride, rows, 1, seqlens ? seqlens : rows + batch, seqlen_add,
+                           out, out_stride_b, out_stride_h, workspace, workspace_bytes, scale,
+                           batch, q_heads, kv_heads, head_dim, 1, max_len, (int)num_firsts,
+                           dtype, num_splits);
   a.contiguous = true;
   a.same_pages = page_size;
   a.q_st = q_stride_t;
@@ -897,7 +886,7 @@ int mxfa_package_contiguous_decode_launch(
       rc = check_split_args(a);
       if (rc != MXFA_OK) return rc;
       RowsParams r{cu_seqlens_q, cu_seqlens_k, cu_q_is_int64, cu_k_is_int64, num_seqs,
-                   num_firsts,   max_len,      batch,         first,         first + batch,
+                   num_firsts,   max_len,      batch,         rows,          rows + batch,
                    host_offsets};
       const size_t lds = cu_seqlens_k ? (size_t)batch * sizeof(int32_t) : 0;
       hipLaunchKernelGGL(contiguous_rows_kernel, dim3(1), dim3(kRowsThreads), lds, st, r);

@@ -15,7 +15,11 @@
 //
 // The workspace is grow-only per (device, stream): a buffer replaced by a
 // larger one stays alive until the process ends, since a HIP graph captured
-// earlier keeps its address.
+// earlier keeps its address. A replay therefore belongs on the stream of the
+// capture, or ordered with it: on another stream, beside eager calls on that
+// one, both write the workspace and give wrong numbers (never a read or write
+// outside the tensors: what the kernels address by is in no workspace, or
+// clamped where it is read).
 //
 // Reference counterpart: the pybind binding paged_decode_split of
 // csrc_native/m1_binding.cpp:78-115 (checks, output and workspace, launch on
@@ -353,8 +357,8 @@ py::object contiguous_decode(const at::Tensor &q, const at::Tensor &k, const at:
   // 33 -> 34.5 us; a dense call 15.2 -> 19.1 us, with the second launch).
   // Asked for the columns of one launch; past 16 columns it is asked again
   // unless it picked the per-sequence kernel.
-  const int64_t rows = packed ? 1 : k.size(1);
-  const int ps = (int)std::min<int64_t>(rows & -rows, 256);
+  const int64_t len = packed ? 1 : k.size(1);
+  const int ps = (int)std::min<int64_t>(len & -len, 256);
   const int cus = num_cus(device.index()), width = (int)((max_len + ps - 1) / ps);
   const int64_t gq = hq / hkv;
   const int64_t first_ask = std::min<int64_t>(ql, std::max<int64_t>(1, 16 / gq));
@@ -371,8 +375,13 @@ py::object contiguous_decode(const at::Tensor &q, const at::Tensor &k, const at:
                                              &ws_bytes) != MXFA_OK)
     return py::none();
   void *stream = (void *)c10::hip::getCurrentHIPStream(device.index()).stream();
-  at::Tensor ws = workspace(device, stream, ws_bytes);
-  poison(stream, out, &ws);
+  at::Tensor ws_t;
+  if (ws_bytes) ws_t = workspace(device, stream, ws_bytes);
+  void *ws = ws_bytes ? ws_t.data_ptr() : nullptr;
+  poison(stream, out, ws_bytes ? &ws_t : nullptr);
+  // First rows and lengths: memory of this call, not the workspace, which
+  // captured graphs write whenever they are replayed.
+  at::Tensor rows_t = at::empty({2 * batch}, q.options().dtype(at::kInt));
   const int64_t token_stride = k.stride(packed ? 0 : 1);
   int64_t *host_offsets = nullptr;
   if (offsets) {
@@ -386,9 +395,9 @@ py::object contiguous_decode(const at::Tensor &q, const at::Tensor &k, const at:
   const int rc = mxfa_package_contiguous_decode_launch(
       q.data_ptr(), qs[0], qs[1], qs[2], (int)ql, causal, k.data_ptr(), v.data_ptr(), k.stride(0),
       token_stride, k.stride(-2), firsts, (int)max_len, cu_q, cu_q64, cu_k, cu_k64, (int)num_seqs,
-      host_offsets, offsets ? offsets->event() : nullptr, seqlens, 0, out.data_ptr(), os[0],
-      os[1], os[2], ws.data_ptr(), ws_bytes, (float)scale, (int)batch, (int)hq, (int)hkv, (int)hd,
-      ps, dt == at::kBFloat16 ? MXFA_DTYPE_BF16 : MXFA_DTYPE_F16, ns, stream);
+      rows_t.data_ptr<int32_t>(), host_offsets, offsets ? offsets->event() : nullptr, seqlens, 0,
+      out.data_ptr(), os[0], os[1], os[2], ws, ws_bytes, (float)scale, (int)batch, (int)hq,
+      (int)hkv, (int)hd, ps, dt == at::kBFloat16 ? MXFA_DTYPE_BF16 : MXFA_DTYPE_F16, ns, stream);
   if (rc == MXFA_EUNSUPPORTED || rc == MXFA_EINVAL) return py::none();  // nothing launched
   if (offsets) {
     if (rc != MXFA_OK) (void)hipStreamSynchronize((hipStream_t)stream);  // no event to wait for

@@ -280,7 +280,9 @@ class _Workspace:
     the smaller one is therefore never released: it moves to a keep-alive list
     for the life of the process, so replays of earlier captures still write
     into memory that nothing else owns. Growth doubles, so the retired buffers
-    together stay smaller than the live one.
+    together stay smaller than the live one. A replay belongs on the stream of
+    the capture, or ordered with it: beside eager calls on that stream both
+    write the workspace and give wrong numbers.
     """
 
     def __init__(self) -> None:

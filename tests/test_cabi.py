@@ -483,3 +483,15 @@ def test_no_alloc_entry_refuses_oversized_and_invalid_calls_before_launch(lib):
     assert fn(*args) == native.MXFA_ESCRATCH
     args[16] = 0  # batch
     assert fn(*args) == native.MXFA_EINVAL
+
+
+@pytest.mark.parametrize("batch,hq,hkv,ql,hd,ns,tokens", [(32, 32, 8, 1, 128, 256, 1),
+                                                          (4, 8, 2, 16, 64, 37, 16),
+                                                          (5, 8, 8, 3, 64, -1, 3)])
+def test_first_rows_and_lengths_are_in_no_workspace(lib, batch, hq, hkv, ql, hd, ns, tokens):
+    # Keys in consecutive rows: what the decode addresses by must not lie in the
+    # workspace, which a replay of a graph captured on the stream also writes.
+    got = ctypes.c_size_t()
+    assert lib.mxfa_package_contiguous_workspace_size(batch, hq, hkv, ql, hd, ns,
+                                                      ctypes.byref(got)) == 0
+    assert got.value == native.workspace_size(batch, hq * tokens, hd, ns)
