@@ -516,6 +516,9 @@ py::object decode_tokens(const at::Tensor &q, const at::Tensor &k_cache, const a
     strides(out, os);
   }
   const bool extras = window_left >= 0 || softcap > 0 || sink_ptr || alibi_ptr;
+  // Only the entry point of several tokens or options takes shortened sequences;
+  // one plain token is refused by the C ABI (mxfa_split_decode_launch).
+  if (seqlen_add < 0 && ql == 1 && !extras) return py::none();
   const int width = (int)block_table.size(1), cus = num_cus(device.index());
   const int64_t wide = mxfa_package_launch_columns((int)hd, (int)ps, fp8, extras);
   const auto heuristic = [&](int64_t columns, int &ns) {

@@ -146,3 +146,26 @@ def test_reshape_and_cache_operator_equals_ctypes_path(device, monkeypatch):
     keep = slots >= 0
     assert torch.equal(kc[slots[keep]], key[keep])
     assert int((kc.abs().sum((1, 2)) > 0).sum()) == int(keep.sum())
+
+
+@pytest.mark.parametrize("fp8", [False, True], ids=["bf16", "fp8"])
+def test_shortened_sequences_are_for_several_tokens_or_options(device, monkeypatch, fp8):
+    """seqlen_add below 0: refused for one plain token and taken otherwise,
+    whether or not the operator is there."""
+    b = make_paged_batch(3, 8, 2, 64, torch.bfloat16, torch.tensor([40, 3, 90]), q_len=2,
+                         seed=4).to(device)
+    kc, vc = (c.to(torch.float8_e4m3fn) if fp8 else c for c in (b.k_cache, b.v_cache))
+
+    def call(q, **kw):
+        return native.paged_decode_split(q, kc, vc, b.block_table, b.cache_seqlens, b.scale,
+                                         seqlen_add=-2, **kw)
+
+    got = {}
+    for op in (True, False):
+        monkeypatch.setattr(native, "USE_TORCH_OP", op)
+        for q in (b.q[:, :1], b.q[:, 0]):
+            with pytest.raises(RuntimeError, match=r"failed \(-2\)"):
+                call(q)
+        got[op] = [call(b.q, causal=True), call(b.q[:, :1], window_left=20)]
+    for a, c in zip(got[True], got[False]):
+        assert torch.isfinite(a.float()).all() and torch.equal(a, c)
