@@ -16,6 +16,19 @@ extern "C" {
 // cap, sinks or ALiBi.
 int mxfa_package_launch_columns(int head_dim, int page_size, int fp8, int extras);
 
+// Query tokens of each launch of a call of q_len tokens when a launch takes
+// `columns`: as many as fit, or, of launches of several column groups, about
+// equal shares (64 columns at head dim 128 are two launches of two groups rather
+// than one of three and one of one).
+int mxfa_package_tokens_per_launch(int q_len, int gq, int columns);
+
+// num_splits for a call of q_len tokens whose launches take `columns`: the
+// heuristic's choice for the columns of one launch of one group, or, where that
+// is the split kernel and launches are of several groups, for one of those.
+int mxfa_package_num_splits(int batch, int q_len, int q_heads, int kv_heads, int head_dim,
+                            int page_size, int block_table_width, int fp8, int columns,
+                            int num_cus, int *num_splits);
+
 // mxfa_split_decode_multi_launch (same arguments, checks and results) for up
 // to mxfa_package_launch_columns columns: every 16 columns past the first are
 // another column group of the same wave, so the keys are read once for all.

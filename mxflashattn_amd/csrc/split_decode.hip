@@ -622,15 +622,16 @@ __global__ __launch_bounds__(kRowsThreads) void contiguous_rows_kernel(RowsParam
   }
 }
 
-// Query tokens of one launch of a contiguous call: all of them, or for a
-// causal query of more columns as many as fit (about equal shares where a
-// launch takes several column groups).
-static int contiguous_tokens(int ql, int gq, int hd, int ns) {
-  const int cols = ns > 0 ? launch_columns(hd, kTile, false, false) : kMaxCols;
-  const int most = cols / gq;
-  if (ql <= most || cols == kMaxCols) return ql < most ? ql : most;
+static int tokens_per_launch(int ql, int gq, int columns) {
+  const int most = columns / gq < 1 ? 1 : columns / gq;
+  if (columns <= kMaxCols) return ql < most ? ql : most;
   const int launches = (ql + most - 1) / most;
   return (ql + launches - 1) / launches;
+}
+
+// Query tokens of one launch of a contiguous call.
+static int contiguous_tokens(int ql, int gq, int hd, int ns) {
+  return tokens_per_launch(ql, gq, ns > 0 ? launch_columns(hd, kTile, false, false) : kMaxCols);
 }
 
 }  // namespace mxfa
@@ -898,6 +899,27 @@ int mxfa_package_contiguous_decode_launch(
     if (rc != MXFA_OK) return rc;
   }
   return MXFA_OK;
+}
+
+int mxfa_package_tokens_per_launch(int q_len, int gq, int columns) {
+  return q_len > 0 && gq > 0 ? tokens_per_launch(q_len, gq, columns) : 0;
+}
+
+int mxfa_package_num_splits(int batch, int q_len, int q_heads, int kv_heads, int head_dim,
+                            int page_size, int block_table_width, int fp8, int columns,
+                            int num_cus, int *num_splits) {
+  if (q_len <= 0 || q_heads <= 0 || kv_heads <= 0) return MXFA_EINVAL;
+  const int gq = q_heads < kv_heads ? 1 : q_heads / kv_heads;
+  const auto ask = [&](int tokens) {
+    return split_heuristic(batch, q_heads * tokens, kv_heads, head_dim, fp8 ? 1 : 2, page_size,
+                           block_table_width, num_cus, num_splits);
+  };
+  const int one = tokens_per_launch(q_len, gq, kMaxCols);
+  const int rc = ask(one);
+  if (rc != MXFA_OK || one == q_len || columns <= kMaxCols ||
+      *num_splits == MXFA_SPLITS_PER_SEQUENCE)
+    return rc;
+  return ask(tokens_per_launch(q_len, gq, columns));
 }
 
 int mxfa_package_launch_columns(int head_dim, int page_size, int fp8, int extras) {

@@ -353,22 +353,14 @@ py::object contiguous_decode(const at::Tensor &q, const at::Tensor &k, const at:
   // maximum: the largest weight of a tile is then no longer exactly 1 before P
   // is rounded, and the error against 64 bits grew by up to 19 % (fp16, HD 64,
   // 8q/2kv, sequences of 500-767 keys: 2.45e-4 -> 2.87e-4; bf16 1.96e-3 ->
-  // 2.30e-3). Splitting them costs 1-4 us a call (5 packed sequences and up:
-  // 33 -> 34.5 us; a dense call 15.2 -> 19.1 us, with the second launch).
-  // Asked for the columns of one launch; past 16 columns it is asked again
-  // unless it picked the per-sequence kernel.
+  // 2.30e-3). The split kernel and its second launch cost 1-4 us a call there (32
+  // packed sequences 33.0 -> 34.5 us, 4 dense ones 15.2 -> 19.1 us).
   const int64_t len = packed ? 1 : k.size(1);
-  const int ps = (int)std::min<int64_t>(len & -len, 256);
-  const int cus = num_cus(device.index()), width = (int)((max_len + ps - 1) / ps);
-  const int64_t gq = hq / hkv;
-  const int64_t first_ask = std::min<int64_t>(ql, std::max<int64_t>(1, 16 / gq));
+  const int ps = (int)std::min<int64_t>(len & -len, 256), width = (int)((max_len + ps - 1) / ps);
   int ns = 0;
-  if (mxfa_split_heuristic((int)batch, (int)(hq * first_ask), (int)hkv, (int)hd, ps, width, cus,
-                           &ns) != MXFA_OK)
-    return py::none();
-  if (first_ask < ql && ns != MXFA_SPLITS_PER_SEQUENCE &&
-      mxfa_split_heuristic((int)batch, (int)(hkv * 17), (int)hkv, (int)hd, ps, width, cus, &ns) !=
-          MXFA_OK)
+  if (mxfa_package_num_splits((int)batch, (int)ql, (int)hq, (int)hkv, (int)hd, ps, width, 0,
+                              mxfa_package_launch_columns((int)hd, 16, 0, 0),
+                              num_cus(device.index()), &ns) != MXFA_OK)
     return py::none();
   size_t ws_bytes = 0;
   if (mxfa_package_contiguous_workspace_size((int)batch, (int)hq, (int)hkv, (int)ql, (int)hd, ns,
@@ -519,33 +511,20 @@ py::object decode_tokens(const at::Tensor &q, const at::Tensor &k_cache, const a
   // Only the entry point of several tokens or options takes shortened sequences;
   // one plain token is refused by the C ABI (mxfa_split_decode_launch).
   if (seqlen_add < 0 && ql == 1 && !extras) return py::none();
-  const int width = (int)block_table.size(1), cus = num_cus(device.index());
-  const int64_t wide = mxfa_package_launch_columns((int)hd, (int)ps, fp8, extras);
-  const auto heuristic = [&](int64_t columns, int &ns) {
-    const auto f = fp8 ? mxfa_split_heuristic_fp8 : mxfa_split_heuristic;
-    return f((int)batch, (int)(hkv * columns), (int)hkv, (int)hd, (int)ps, width, cus, &ns) ==
-           MXFA_OK;
-  };
-  // num_splits as the Python binding's default_num_splits chooses it: asked for
-  // the columns of one launch, then, past 16 of them and unless the
-  // per-sequence kernel was picked, for a launch of several column groups.
+  const int width = (int)block_table.size(1);
+  const int wide = mxfa_package_launch_columns((int)hd, (int)ps, fp8, extras);
   int ns = 0;
   if (num_splits_arg.has_value()) {
     const int64_t v = *num_splits_arg;
     if ((v <= 0 && v != MXFA_SPLITS_PER_SEQUENCE) || v > 65535) return py::none();
     ns = (int)v;
-  } else {
-    if (!heuristic(gq * std::min<int64_t>(ql, 16 / gq), ns)) return py::none();
-    if (ql > 16 / gq && ns != MXFA_SPLITS_PER_SEQUENCE && wide > 16 && !heuristic(17, ns))
-      return py::none();
+  } else if (mxfa_package_num_splits((int)batch, (int)ql, (int)hq, (int)hkv, (int)hd, (int)ps,
+                                     width, fp8, wide, num_cus(device.index()), &ns) !=
+             MXFA_OK) {
+    return py::none();
   }
-  // Tokens per launch (native.tokens_per_launch).
-  const int64_t columns = ql * gq > 16 && ns != MXFA_SPLITS_PER_SEQUENCE ? wide : 16;
-  int64_t tokens = std::min<int64_t>(ql, columns / gq);
-  if (columns > 16) {
-    const int64_t launches = (ql + tokens - 1) / tokens;
-    tokens = (ql + launches - 1) / launches;
-  }
+  const int64_t tokens = mxfa_package_tokens_per_launch(
+      (int)ql, (int)gq, ns == MXFA_SPLITS_PER_SEQUENCE ? 16 : wide);
   size_t ws_bytes = 0;
   if (mxfa_split_decode_workspace_size((int)batch, (int)(hq * tokens), (int)hd, ns, &ws_bytes) !=
       MXFA_OK)

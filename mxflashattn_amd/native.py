@@ -151,6 +151,8 @@ _SIGNATURES = {
 # Entry points for this package only (csrc/mxfa_package.h), not part of the C ABI.
 _PACKAGE_SIGNATURES = {
     "mxfa_package_launch_columns": (_i, [_i, _i, _i, _i]),
+    "mxfa_package_tokens_per_launch": (_i, [_i, _i, _i]),
+    "mxfa_package_num_splits": (_i, [*[_i] * 10, _p]),
     "mxfa_package_decode_tokens_launch": (
         _i, [*_SIGNATURES["mxfa_split_decode_multi_launch"][1][:-1], _p, _i, _p]),
 }
@@ -589,12 +591,8 @@ def launch_columns(head_dim: int, page_size: int, fp8: bool, extras: bool) -> in
 
 def tokens_per_launch(q_len: int, gq: int, columns: int) -> int:
     """Query tokens of each launch: as many as ``columns`` hold, or, of launches
-    of several column groups, about equal shares (64 columns at head dim 128
-    are two launches of two groups rather than one of three and one of one)."""
-    if columns <= KERNEL_COLUMNS:
-        return min(q_len, columns // gq)
-    launches = -(-q_len // (columns // gq))
-    return -(-q_len // launches)
+    of several column groups, about equal shares."""
+    return library().mxfa_package_tokens_per_launch(q_len, gq, columns)
 
 
 def _sinks_ptr(values, q: torch.Tensor, name: str = "sinks") -> int:
@@ -611,26 +609,20 @@ def _sinks_ptr(values, q: torch.Tensor, name: str = "sinks") -> int:
 
 
 def default_num_splits(q: torch.Tensor, k_cache: torch.Tensor, block_table: torch.Tensor) -> int:
-    """The heuristic's count for q ([B, HQ, HD] or [B, QL, HQ, HD]). It is
-    asked for the columns of one launch, HQ times the query tokens a launch
-    takes (QL, or for longer causal queries 16 / GQ of them), which decide
-    whether the per-sequence kernel's LDS holds them; a causal query past 16
-    columns that it gives to the split kernel asks again for the columns that
-    kernel takes at once."""
-    hq, hkv = q.shape[-2], k_cache.shape[2]
-    gq = max(1, hq // hkv)
-    ql = q.shape[1] if q.dim() == 4 else 1
+    """The heuristic's count for q ([B, HQ, HD] or [B, QL, HQ, HD])."""
     fp8 = k_cache.dtype == FP8_DTYPE
-    batch, hd, ps, width = q.shape[0], q.shape[-1], k_cache.shape[1], block_table.shape[1]
-    cus = num_cus(q.device.index or 0)
-    tokens = min(ql, max(1, KERNEL_COLUMNS // gq))
-    ns = split_heuristic(batch, hq * tokens, hkv, hd, ps, width, cus, fp8)
-    if ql > tokens and ns != SPLITS_PER_SEQUENCE:
-        columns = launch_columns(hd, ps, fp8, False)
-        if columns > KERNEL_COLUMNS:
-            ns = split_heuristic(batch, hq * tokens_per_launch(ql, gq, columns), hkv, hd, ps,
-                                 width, cus, fp8)
-    return ns
+    return _num_splits(q.shape[0], q.shape[1] if q.dim() == 4 else 1, q.shape[-2],
+                       k_cache.shape[2], q.shape[-1], k_cache.shape[1], block_table.shape[1], fp8,
+                       launch_columns(q.shape[-1], k_cache.shape[1], fp8, False),
+                       num_cus(q.device.index or 0))
+
+
+@functools.lru_cache(maxsize=256)
+def _num_splits(*args: int) -> int:
+    """mxfa_package_num_splits of its arguments."""
+    ns = _i()
+    _check(library().mxfa_package_num_splits(*args, ctypes.byref(ns)), "mxfa_package_num_splits")
+    return ns.value
 
 
 def _op_scales(*values) -> bool:

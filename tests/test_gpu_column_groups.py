@@ -68,6 +68,27 @@ def test_column_groups_round_no_more_than_launches_of_16_columns(device, head_di
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("head_dim,gq,ql", [(64, 2, 12), (64, 4, 16), (128, 4, 16), (128, 1, 17)])
+@pytest.mark.parametrize("width", [16, 128])  # the per-sequence kernel, the split kernel
+@pytest.mark.parametrize("fp8", [False, True], ids=["bf16", "fp8"])
+def test_operator_splits_as_the_binding(device, monkeypatch, head_dim, gq, ql, width, fp8):
+    b = make_paged_batch(6, 8 * gq, 8, head_dim, torch.bfloat16, torch.arange(6) * 40 + ql,
+                         q_len=ql, block_table_width=width, seed=ql).to(device)
+    kc, vc = (c.to(FP8) if fp8 else c for c in (b.k_cache, b.v_cache))
+
+    def call():
+        return native.paged_decode_split(b.q, kc, vc, b.block_table, b.cache_seqlens, b.scale,
+                                         causal=True)
+
+    assert native.torch_op().decode_tokens(b.q, kc, vc, b.block_table, b.cache_seqlens, b.scale,
+                                           None, None, 0, True, -1, 0.0, None, None, None,
+                                           None) is not None
+    out = call()
+    monkeypatch.setattr(native, "USE_TORCH_OP", False)
+    assert torch.equal(out, call())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("head_dim", [64, 128])
 @pytest.mark.parametrize("ql,gq", [(17, 1), (31, 1), (16, 2), (11, 3), (33, 1), (47, 1), (12, 4),
                                    (49, 1), (9, 7), (64, 1), (4, 16)])
