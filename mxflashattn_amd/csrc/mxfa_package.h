@@ -59,15 +59,16 @@ int mxfa_package_decode_tokens_launch(
 //     write, or null) receives cu_q then cu_k; offsets_event (a hipEvent_t, or
 //     null) is recorded once they are there, ahead of the decode.
 // rows (2 * batch int32 in device memory): one small launch writes first rows
-// and lengths there, and the decode reads them. Memory of this call alone: first
+// and lengths there (unless rows_written: an earlier launch of the same call
+// did), and the decode reads them. Memory of this call alone: first
 // rows and lengths are held to the rows that exist where they are written, so
 // nothing else (a replay of a graph that holds a workspace) may write them
 // before the decode has read them.
 // page_size: of the pages that hold the same bytes (1 for packed keys); with the
 // splits their heuristic chooses, one token's result is that of those pages.
-// Any number of causal query tokens, as many per launch as the kernel takes.
-// Workspace from mxfa_package_contiguous_workspace_size (none for
-// MXFA_SPLITS_PER_SEQUENCE).
+// q_len query tokens of at most mxfa_package_launch_columns(head_dim, 16, 0, 0)
+// columns; mxfa_package_contiguous_workspace_size is the workspace of the widest
+// launch of a call of q_len tokens (0 for MXFA_SPLITS_PER_SEQUENCE).
 int mxfa_package_contiguous_workspace_size(int batch, int q_heads, int kv_heads, int q_len,
                                            int head_dim, int num_splits, size_t *bytes);
 int mxfa_package_contiguous_decode_launch(
@@ -75,10 +76,11 @@ int mxfa_package_contiguous_decode_launch(
     int causal, const void *k, const void *v, int64_t first_stride, int64_t token_stride,
     int64_t head_stride, int64_t num_firsts, int max_len, const void *cu_seqlens_q,
     int cu_q_is_int64, const void *cu_seqlens_k, int cu_k_is_int64, int num_seqs,
-    int32_t *rows, int64_t *host_offsets, void *offsets_event, const int32_t *seqlens,
-    int seqlen_add, void *out, int64_t out_stride_b, int64_t out_stride_t, int64_t out_stride_h,
-    void *workspace, size_t workspace_bytes, float scale, int batch, int q_heads, int kv_heads,
-    int head_dim, int page_size, int dtype, int num_splits, void *stream);
+    int32_t *rows, int rows_written, int64_t *host_offsets, void *offsets_event,
+    const int32_t *seqlens, int seqlen_add, void *out, int64_t out_stride_b, int64_t out_stride_t,
+    int64_t out_stride_h, void *workspace, size_t workspace_bytes, float scale, int batch,
+    int q_heads, int kv_heads, int head_dim, int page_size, int dtype, int num_splits,
+    void *stream);
 
 #ifdef __cplusplus
 }

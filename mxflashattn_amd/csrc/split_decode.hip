@@ -847,21 +847,16 @@ int mxfa_package_contiguous_decode_launch(
     int causal, const void *k, const void *v, int64_t first_stride, int64_t token_stride,
     int64_t head_stride, int64_t num_firsts, int max_len, const void *cu_seqlens_q,
     int cu_q_is_int64, const void *cu_seqlens_k, int cu_k_is_int64, int num_seqs,
-    int32_t *rows, int64_t *host_offsets, void *offsets_event, const int32_t *seqlens,
-    int seqlen_add, void *out, int64_t out_stride_b, int64_t out_stride_t, int64_t out_stride_h,
-    void *workspace, size_t workspace_bytes, float scale, int batch, int q_heads, int kv_heads,
-    int head_dim, int page_size, int dtype, int num_splits, void *stream) {
-  size_t need = 0;
-  int rc = mxfa_package_contiguous_workspace_size(batch, q_heads, kv_heads, q_len, head_dim,
-                                                  num_splits, &need);
-  if (rc != MXFA_OK) return rc;
-  if (workspace_bytes < need) return MXFA_EWORKSPACE;
-  if (!rows || ((uintptr_t)rows & 3u)) return MXFA_EINVAL;
-  if (num_firsts <= 0 || num_firsts > INT32_MAX || max_len <= 0) return MXFA_EINVAL;
+    int32_t *rows, int rows_written, int64_t *host_offsets, void *offsets_event,
+    const int32_t *seqlens, int seqlen_add, void *out, int64_t out_stride_b, int64_t out_stride_t,
+    int64_t out_stride_h, void *workspace, size_t workspace_bytes, float scale, int batch,
+    int q_heads, int kv_heads, int head_dim, int page_size, int dtype, int num_splits,
+    void *stream) {
+  if (!rows || ((uintptr_t)rows & 3u) || num_firsts <= 0 || num_firsts > INT32_MAX ||
+      max_len <= 0)
+    return MXFA_EINVAL;
   if (cu_seqlens_k ? (!cu_seqlens_q || num_seqs < batch || seqlens) : num_firsts < batch)
     return MXFA_EINVAL;
-  const int tokens = contiguous_tokens(q_len, q_heads / kv_heads, head_dim, num_splits);
-  if (tokens < q_len && !causal) return MXFA_EUNSUPPORTED;
   SplitArgs a = split_args(q, q_stride_b, q_stride_h, k, v, first_stride, token_stride,
                            head_stride, rows, 1, seqlens ? seqlens : rows + batch, seqlen_add,
                            out, out_stride_b, out_stride_h, workspace, workspace_bytes, scale,
@@ -871,34 +866,24 @@ int mxfa_package_contiguous_decode_launch(
   a.same_pages = page_size;
   a.q_st = q_stride_t;
   a.o_st = out_stride_t;
+  a.ql = q_len;
   a.causal = causal;
   a.min_seqlen_add = -(1 << 30);
   if (num_splits > 0) a.max_cols = launch_columns(head_dim, kTile, false, false);
+  const int rc = check_split_args(a);
+  if (rc != MXFA_OK) return rc;
   const hipStream_t st = (hipStream_t)stream;
-  // A causal query of several launches: tokens [t, t + n) run as the last n
-  // tokens of sequences shortened by the tokens after them.
-  for (int t = 0; t < q_len; t += tokens) {
-    const int n = q_len - t < tokens ? q_len - t : tokens;
-    a.q = (const char *)q + (int64_t)t * q_stride_t * 2;
-    a.out = (char *)out + (int64_t)t * out_stride_t * 2;
-    a.ql = n;
-    a.seqlen_add = seqlen_add - (q_len - t - n);
-    if (t == 0) {
-      rc = check_split_args(a);
-      if (rc != MXFA_OK) return rc;
-      RowsParams r{cu_seqlens_q, cu_seqlens_k, cu_q_is_int64, cu_k_is_int64, num_seqs,
-                   num_firsts,   max_len,      batch,         rows,          rows + batch,
-                   host_offsets};
-      const size_t lds = cu_seqlens_k ? (size_t)batch * sizeof(int32_t) : 0;
-      hipLaunchKernelGGL(contiguous_rows_kernel, dim3(1), dim3(kRowsThreads), lds, st, r);
-      if (hipGetLastError() != hipSuccess) return MXFA_ELAUNCH;
-      if (offsets_event && hipEventRecord((hipEvent_t)offsets_event, st) != hipSuccess)
-        return MXFA_ELAUNCH;
-    }
-    rc = run_split(a, true, st);
-    if (rc != MXFA_OK) return rc;
+  if (!rows_written) {
+    RowsParams r{cu_seqlens_q, cu_seqlens_k, cu_q_is_int64, cu_k_is_int64, num_seqs,
+                 num_firsts,   max_len,      batch,         rows,          rows + batch,
+                 host_offsets};
+    const size_t lds = cu_seqlens_k ? (size_t)batch * sizeof(int32_t) : 0;
+    hipLaunchKernelGGL(contiguous_rows_kernel, dim3(1), dim3(kRowsThreads), lds, st, r);
+    if (hipGetLastError() != hipSuccess) return MXFA_ELAUNCH;
+    if (offsets_event && hipEventRecord((hipEvent_t)offsets_event, st) != hipSuccess)
+      return MXFA_ELAUNCH;
   }
-  return MXFA_OK;
+  return run_split(a, true, st);
 }
 
 int mxfa_package_tokens_per_launch(int q_len, int gq, int columns) {

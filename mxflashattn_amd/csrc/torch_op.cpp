@@ -75,9 +75,9 @@ at::Tensor workspace(const at::Device &device, void *stream, size_t bytes) {
 }
 
 // MXFA_POISON_OUTPUTS=1 (a debugging aid, read once; the Python binding reads
-// the same variable): before each launch outside graph capture the output is
-// filled with NaN and the workspace with 0xff bytes, so a row or a piece the
-// kernels fail to write shows up as NaN rather than as a stale value.
+// the same variable): outside graph capture the output of a call is filled with
+// NaN and the workspace of each of its launches with 0xff bytes, so a row or a
+// piece the kernels fail to write shows up as NaN rather than as a stale value.
 bool poison_outputs() {
   static const bool on = [] {
     const char *e = std::getenv("MXFA_POISON_OUTPUTS");
@@ -86,14 +86,14 @@ bool poison_outputs() {
   return on;
 }
 
-void poison(void *stream, at::Tensor &out, at::Tensor *ws) {
+void poison(void *stream, at::Tensor *out, at::Tensor *ws) {
   // An output whose rows overlap is refused by the launch; it is not filled.
-  if (!poison_outputs() || at::has_internal_overlap(out) != at::MemOverlap::No) return;
+  if (!poison_outputs() || (out && at::has_internal_overlap(*out) != at::MemOverlap::No)) return;
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing((hipStream_t)stream, &status) != hipSuccess ||
       status != hipStreamCaptureStatusNone)
     return;
-  out.fill_(std::numeric_limits<float>::quiet_NaN());
+  if (out) out->fill_(std::numeric_limits<float>::quiet_NaN());
   if (ws) ws->fill_(0xff);
 }
 
@@ -200,7 +200,7 @@ py::object decode(const at::Tensor &q, const at::Tensor &k_cache, const at::Tens
   at::Tensor ws_t;
   if (ws_bytes) ws_t = workspace(device, stream, ws_bytes);
   void *ws = ws_bytes ? ws_t.data_ptr() : nullptr;
-  poison(stream, out, ws_bytes ? &ws_t : nullptr);
+  poison(stream, &out, ws_bytes ? &ws_t : nullptr);
   const int rc = mxfa_split_decode_launch(
       q.data_ptr(), q_sb, q_sh, k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0),
       k_cache.stride(1), k_cache.stride(2), block_table.data_ptr<int32_t>(), block_table.stride(0),
@@ -357,11 +357,14 @@ py::object contiguous_decode(const at::Tensor &q, const at::Tensor &k, const at:
   // packed sequences 33.0 -> 34.5 us, 4 dense ones 15.2 -> 19.1 us).
   const int64_t len = packed ? 1 : k.size(1);
   const int ps = (int)std::min<int64_t>(len & -len, 256), width = (int)((max_len + ps - 1) / ps);
+  const int wide = mxfa_package_launch_columns((int)hd, 16, 0, 0);
   int ns = 0;
-  if (mxfa_package_num_splits((int)batch, (int)ql, (int)hq, (int)hkv, (int)hd, ps, width, 0,
-                              mxfa_package_launch_columns((int)hd, 16, 0, 0),
+  if (mxfa_package_num_splits((int)batch, (int)ql, (int)hq, (int)hkv, (int)hd, ps, width, 0, wide,
                               num_cus(device.index()), &ns) != MXFA_OK)
     return py::none();
+  const int64_t tokens = mxfa_package_tokens_per_launch(
+      (int)ql, (int)(hq / hkv), ns == MXFA_SPLITS_PER_SEQUENCE ? 16 : wide);
+  if (tokens < ql && !causal) return py::none();
   size_t ws_bytes = 0;
   if (mxfa_package_contiguous_workspace_size((int)batch, (int)hq, (int)hkv, (int)ql, (int)hd, ns,
                                              &ws_bytes) != MXFA_OK)
@@ -370,7 +373,7 @@ py::object contiguous_decode(const at::Tensor &q, const at::Tensor &k, const at:
   at::Tensor ws_t;
   if (ws_bytes) ws_t = workspace(device, stream, ws_bytes);
   void *ws = ws_bytes ? ws_t.data_ptr() : nullptr;
-  poison(stream, out, ws_bytes ? &ws_t : nullptr);
+  poison(stream, &out, ws_bytes ? &ws_t : nullptr);
   // First rows and lengths: memory of this call, not the workspace, which
   // captured graphs write whenever they are replayed.
   at::Tensor rows_t = at::empty({2 * batch}, q.options().dtype(at::kInt));
@@ -384,20 +387,29 @@ py::object contiguous_decode(const at::Tensor &q, const at::Tensor &k, const at:
         !(host_offsets = offsets->memory()))
       return py::none();
   }
-  const int rc = mxfa_package_contiguous_decode_launch(
-      q.data_ptr(), qs[0], qs[1], qs[2], (int)ql, causal, k.data_ptr(), v.data_ptr(), k.stride(0),
-      token_stride, k.stride(-2), firsts, (int)max_len, cu_q, cu_q64, cu_k, cu_k64, (int)num_seqs,
-      rows_t.data_ptr<int32_t>(), host_offsets, offsets ? offsets->event() : nullptr, seqlens, 0,
-      out.data_ptr(), os[0], os[1], os[2], ws, ws_bytes, (float)scale, (int)batch, (int)hq,
-      (int)hkv, (int)hd, ps, dt == at::kBFloat16 ? MXFA_DTYPE_BF16 : MXFA_DTYPE_F16, ns, stream);
-  if (rc == MXFA_EUNSUPPORTED || rc == MXFA_EINVAL) return py::none();  // nothing launched
-  if (offsets) {
-    if (rc != MXFA_OK) (void)hipStreamSynchronize((hipStream_t)stream);  // no event to wait for
-    else offsets->launched();
+  for (int64_t t = 0; t < ql; t += tokens) {
+    const int64_t n = std::min(tokens, ql - t);
+    if (t > 0) poison(stream, nullptr, ws_bytes ? &ws_t : nullptr);
+    // Tokens [t, t + n) as the last n tokens of sequences shortened by the
+    // tokens after them.
+    const int rc = mxfa_package_contiguous_decode_launch(
+        (const char *)q.data_ptr() + t * qs[1] * 2, qs[0], qs[1], qs[2], (int)n, causal,
+        k.data_ptr(), v.data_ptr(), k.stride(0), token_stride, k.stride(-2), firsts, (int)max_len,
+        cu_q, cu_q64, cu_k, cu_k64, (int)num_seqs, rows_t.data_ptr<int32_t>(), t > 0,
+        host_offsets, offsets ? offsets->event() : nullptr, seqlens, (int)(t + n - ql),
+        (char *)out.data_ptr() + t * os[1] * 2, os[0], os[1], os[2], ws, ws_bytes, (float)scale,
+        (int)batch, (int)hq, (int)hkv, (int)hd, ps,
+        dt == at::kBFloat16 ? MXFA_DTYPE_BF16 : MXFA_DTYPE_F16, ns, stream);
+    if (t == 0 && (rc == MXFA_EUNSUPPORTED || rc == MXFA_EINVAL))
+      return py::none();  // nothing launched
+    if (offsets) {  // one token
+      if (rc != MXFA_OK) (void)hipStreamSynchronize((hipStream_t)stream);  // no event to wait for
+      else offsets->launched();
+    }
+    if (rc != MXFA_OK)
+      throw std::runtime_error(std::string("contiguous decode failed (") + std::to_string(rc) +
+                               "): " + mxfa_strerror(rc));
   }
-  if (rc != MXFA_OK)
-    throw std::runtime_error(std::string("contiguous decode failed (") + std::to_string(rc) +
-                             "): " + mxfa_strerror(rc));
   return py::cast(out);
 }
 
@@ -533,10 +545,11 @@ py::object decode_tokens(const at::Tensor &q, const at::Tensor &k_cache, const a
   at::Tensor ws_t;
   if (ws_bytes) ws_t = workspace(device, stream, ws_bytes);
   void *ws = ws_bytes ? ws_t.data_ptr() : nullptr;
-  poison(stream, out, ws_bytes ? &ws_t : nullptr);
+  poison(stream, &out, ws_bytes ? &ws_t : nullptr);
   const int64_t esz = 2;
   for (int64_t t = 0; t < ql; t += tokens) {
     const int64_t n = std::min(tokens, ql - t);
+    if (t > 0) poison(stream, nullptr, ws_bytes ? &ws_t : nullptr);
     // Tokens [t, t + n) as the last n tokens of sequences shortened by the
     // tokens after them.
     const int rc = mxfa_package_decode_tokens_launch(

@@ -135,3 +135,33 @@ def test_column_groups_on_both_tile_scans(device, batch):
     out = native.paged_decode_split(d.q, d.k_cache, d.v_cache, d.block_table, d.cache_seqlens,
                                     d.scale, causal=True, num_splits=100)
     assert (out.float().cpu() - ref).abs().max().item() <= TOL[torch.bfloat16]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("call", ["paged", "dense"])
+def test_poison_fills_the_workspace_of_every_launch(device, call):
+    """16 tokens at GQ 4, head dim 128: two launches, each with a workspace that
+    MXFA_POISON_OUTPUTS (set for the tests) fills first."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Fills(TorchDispatchMode):
+        dtypes = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if func is torch.ops.aten.fill_.Scalar:
+                self.dtypes.append(args[0].dtype)
+            return func(*args, **(kwargs or {}))
+
+    b = make_paged_batch(2, 32, 8, 128, torch.bfloat16, torch.tensor([1040, 1040]), q_len=16,
+                         seed=5).to(device)
+    k, v = (torch.randn(2, 1040, 8, 128, device=device).to(torch.bfloat16) for _ in range(2))
+    op = native.torch_op()
+    Fills.dtypes = []
+    with Fills():
+        if call == "paged":
+            out = op.decode_tokens(b.q, b.k_cache, b.v_cache, b.block_table, b.cache_seqlens,
+                                   b.scale, None, None, 0, True, -1, 0.0, None, None, None, None)
+        else:
+            out = op.contiguous_decode(b.q, k, v, b.scale, True, 1040)
+    assert out is not None and torch.isfinite(out.float()).all()
+    assert Fills.dtypes.count(torch.bfloat16) == 1 and Fills.dtypes.count(torch.uint8) == 2
