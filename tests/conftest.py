@@ -41,6 +41,31 @@ def device():
     return torch.device("cuda", 0)
 
 
+@pytest.fixture
+def taken(monkeypatch):
+    """The operator's calls that took what they were given, by name, in order: an
+    operator call that declines (None or False) leaves the call to another route,
+    which gives the same answer."""
+    from mxflashattn_amd import native
+
+    real, names = native.torch_op(), []
+
+    class Recorder:
+        def __getattr__(self, name):
+            fn = getattr(real, name)
+
+            def call(*args, **kwargs):
+                result = fn(*args, **kwargs)
+                if result is not None and result is not False:
+                    names.append(name)
+                return result
+
+            return call
+
+    monkeypatch.setattr(native, "torch_op", Recorder)
+    return names
+
+
 @pytest.fixture(autouse=True)
 def _announce(request: pytest.FixtureRequest):
     # Name the case on stdout before a GPU test runs, so a run that dies

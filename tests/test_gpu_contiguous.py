@@ -25,21 +25,22 @@ def close(got, expected, dtype):
     assert err <= TOL[dtype], err
 
 
-def both_routes(monkeypatch, call):
-    """The call through the operator and through the paged route."""
+def both_routes(monkeypatch, taken, call):
+    """The call as consecutive rows (the operator takes it) and through the paged route."""
+    taken.clear()
     out = call()
+    assert taken[-1] == "contiguous_decode"
     assert mx.get_last_dispatch_info().backend == mx.BACKEND_MI355X
-    monkeypatch.setattr(native, "USE_TORCH_OP", False)
-    paged = call()
-    monkeypatch.undo()
-    return out, paged
+    with monkeypatch.context() as m:
+        m.setattr(native, "USE_TORCH_OP", False)
+        return out, call()
 
 
 @pytest.mark.parametrize("hd,gq,dtype", [(64, 1, torch.float16), (64, 8, torch.bfloat16),
                                          (128, 2, torch.float16), (128, 4, torch.bfloat16),
                                          (128, 16, torch.bfloat16)])
 @pytest.mark.parametrize("wide", [False, True], ids=["int32", "int64"])
-def test_packed_rows(device, monkeypatch, hd, gq, dtype, wide):
+def test_packed_rows(device, monkeypatch, taken, hd, gq, dtype, wide):
     hkv = 3
     lens = [1, 15, 16, 17, 700, 33, 1900, 5]
     rows = [1, 1, 0, 1, 1, 0, 1, 1]  # sequences 2 and 5 have no query row
@@ -53,14 +54,14 @@ def test_packed_rows(device, monkeypatch, hd, gq, dtype, wide):
     d = kv.to(device)
     qd = torch.empty(sum(rows), hkv * gq + 1, hd, dtype=dtype, device=device)
     qd[:, 1:] = q.to(device)
-    out, paged = both_routes(monkeypatch, lambda: mx.flash_attn_varlen_func(
+    out, paged = both_routes(monkeypatch, taken, lambda: mx.flash_attn_varlen_func(
         qd[:, 1:], d[:, 0], d[:, 1], cu_q.to(device, dt), cu_k.to(device, dt), 1, max(lens)))
     close(out, ref, dtype)
     assert torch.equal(out, paged)  # the same tiles, ranges and arithmetic
 
 
 @pytest.mark.parametrize("hd", [64, 128])
-def test_short_packed_sequences_are_split_as_their_pages(device, monkeypatch, hd):
+def test_short_packed_sequences_are_split_as_their_pages(device, monkeypatch, taken, hd):
     # Sequences short enough for the per-sequence kernel, which rounds more
     # weights against one reference maximum: one-token pages never took it.
     lens = [1, 16, 200, 255, 31]
@@ -69,7 +70,7 @@ def test_short_packed_sequences_are_split_as_their_pages(device, monkeypatch, hd
     cu_q, cu_k = torch.arange(6), torch.tensor([0, *torch.tensor(lens).cumsum(0).tolist()])
     ref = reference_port.attention_varlen(q.float(), k.float(), v.float(), cu_q.tolist(),
                                           cu_k.tolist(), softmax_scale=hd ** -0.5)
-    out, paged = both_routes(monkeypatch, lambda: mx.flash_attn_varlen_func(
+    out, paged = both_routes(monkeypatch, taken, lambda: mx.flash_attn_varlen_func(
         q.to(device), k.to(device), v.to(device), cu_q.to(device), cu_k.to(device), 1, 255))
     close(out, ref, torch.float16)
     assert torch.equal(out, paged)
@@ -77,10 +78,10 @@ def test_short_packed_sequences_are_split_as_their_pages(device, monkeypatch, hd
 
 @pytest.mark.parametrize("seq", [33, 129, 250, 383])  # pages of 1 or 2 tokens
 @pytest.mark.parametrize("hd", [64, 128])
-def test_short_odd_dense_keys_are_split_as_their_pages(device, monkeypatch, seq, hd):
+def test_short_odd_dense_keys_are_split_as_their_pages(device, monkeypatch, taken, seq, hd):
     k, v = (randn(4, seq, 2, hd, dtype=torch.bfloat16, seed=s).to(device) for s in (1, 2))
     q = randn(4, 1, 8, hd, dtype=torch.bfloat16, seed=3).to(device)
-    out, paged = both_routes(monkeypatch, lambda: mx.flash_attn_func(q, k, v, causal=True))
+    out, paged = both_routes(monkeypatch, taken, lambda: mx.flash_attn_func(q, k, v, causal=True))
     assert torch.equal(out, paged)
 
 
@@ -88,7 +89,7 @@ def test_short_odd_dense_keys_are_split_as_their_pages(device, monkeypatch, seq,
 @pytest.mark.parametrize("hd,gq,ql,dtype", [(64, 2, 1, torch.float16), (128, 4, 1, torch.bfloat16),
                                             (128, 1, 3, torch.bfloat16), (64, 4, 9, torch.float16),
                                             (128, 4, 16, torch.bfloat16)])
-def test_dense_rows(device, monkeypatch, seq, hd, gq, ql, dtype):
+def test_dense_rows(device, monkeypatch, taken, seq, hd, gq, ql, dtype):
     if ql > seq:
         pytest.skip("fewer keys than query tokens")
     kv = randn(3, seq, 2, 2, hd, dtype=dtype, seed=seq)  # token rows of K and V interleaved
@@ -96,7 +97,7 @@ def test_dense_rows(device, monkeypatch, seq, hd, gq, ql, dtype):
     ref = reference_port.attention_batched(q.float(), kv[:, :, 0].float(), kv[:, :, 1].float(),
                                            softmax_scale=hd ** -0.5, causal=True)
     d = kv.to(device)
-    out, paged = both_routes(monkeypatch, lambda: mx.flash_attn_func(
+    out, paged = both_routes(monkeypatch, taken, lambda: mx.flash_attn_func(
         q.to(device), d[:, :, 0], d[:, :, 1], causal=True))
     close(out, ref, dtype)
     close(paged, ref, dtype)
@@ -108,6 +109,7 @@ def test_dense_rows(device, monkeypatch, seq, hd, gq, ql, dtype):
     got = mx.flash_attn_with_kvcache(q.to(device), d[:, :, 0], d[:, :, 1],
                                      cache_seqlens=lens.to(device), causal=True,
                                      out=buf[:, :, 1:-2])
+    assert taken[-1] == "contiguous_decode"
     assert got.data_ptr() == buf[:, :, 1:-2].data_ptr()
     for b in range(3):
         n = int(lens[b])
@@ -156,7 +158,7 @@ def test_a_row_that_several_sequences_name_takes_one_of_them(device):
         mx.flash_attn_varlen_func(q, k, v, cu_q, cu_k, 1, 100)
 
 
-def test_packed_offsets_are_checked_after_the_launch(device):
+def test_packed_offsets_are_checked_after_the_launch(device, taken):
     """Offsets the API rejects raise the same errors as before the kernels
     went out first, leave the next call right, and name no row outside."""
     k, v = (randn(60, 2, 64, dtype=torch.float16, seed=s).to(device) for s in (8, 9))
@@ -173,11 +175,81 @@ def test_packed_offsets_are_checked_after_the_launch(device):
                               ([0, 2, 2, 3], good, "cu_seqlens_q contains a sequence longer"),
                               ([1, 1, 2, 3], good, "cu_seqlens_q must start at zero"),
                               ([0, 1, 2, 3, 3], good, "same batch size")):
+        taken.clear()
         with pytest.raises(ValueError, match=match):
             call(cu_q, cu_k)
+        # The last one's vectors differ in length: nothing goes out early.
+        assert taken[-1:] == (["contiguous_decode"] if len(cu_q) == 4 else ["PackedOffsets"])
     with pytest.raises(ValueError, match="cu_seqlens_k contains a sequence longer"):
         call([0, 1, 2, 3], good, max_k=38)
+    taken.clear()
     out = call([0, 1, 2, 3], good)
+    assert taken == ["PackedOffsets", "contiguous_decode"]
     ref = reference_port.attention_varlen(q.float().cpu(), k.float().cpu(), v.float().cpu(),
                                           [0, 1, 2, 3], good.tolist(), softmax_scale=0.125)
     close(out, ref, torch.float16)
+
+
+def test_packed_offsets_reach_the_host(device):
+    op = native.torch_op()
+    k, v = (randn(500, 1, 64, dtype=torch.bfloat16, seed=s).to(device) for s in (1, 2))
+    for n, dt in ((3, torch.int32), (250, torch.int64), (3, torch.int64)):
+        q = randn(n, 2, 64, dtype=torch.bfloat16, seed=n).to(device)
+        cu_q = torch.arange(n + 1)
+        cu_k = torch.linspace(0, 500, n + 1).long()
+        offsets = op.PackedOffsets()
+        assert offsets.get() is None
+        out = op.contiguous_decode(q, k, v, 0.125, False, 500, cu_q.to(device, dt),
+                                   cu_k.to(device, dt), offsets=offsets)
+        assert out is not None
+        assert offsets.get() == (cu_q.tolist(), cu_k.tolist())
+
+
+# One lane's, four lanes' and the LDS tile scan; past one pass of the rows launch.
+@pytest.mark.parametrize("seqs", [65, 257, 1100])
+@pytest.mark.parametrize("hd,dtype", [(64, torch.float16), (128, torch.bfloat16)])
+def test_many_sequences(device, monkeypatch, taken, seqs, hd, dtype):
+    g = torch.Generator().manual_seed(seqs)
+    lens = torch.randint(1, 60, (seqs,), generator=g)
+    rows = torch.randint(0, 4, (seqs,), generator=g).clamp(max=1)  # a quarter without a row
+    k, v = (randn(int(lens.sum()), 2, hd, dtype=dtype, seed=s) for s in (1, 2))
+    q = randn(int(rows.sum()), 4, hd, dtype=dtype, seed=3)
+    cu_q, cu_k = (torch.nn.functional.pad(t.cumsum(0), (1, 0)) for t in (rows, lens))
+    ref = reference_port.attention_varlen(q.float(), k.float(), v.float(), cu_q.tolist(),
+                                          cu_k.tolist(), softmax_scale=hd ** -0.5)
+    out, paged = both_routes(monkeypatch, taken, lambda: mx.flash_attn_varlen_func(
+        q.to(device), k.to(device), v.to(device), cu_q.to(device), cu_k.to(device), 1, 59))
+    close(out, ref, dtype)
+    assert torch.equal(out, paged)
+    kd, vd = (randn(seqs, 51, 2, hd, dtype=dtype, seed=s) for s in (4, 5))
+    qd = randn(seqs, 1, 4, hd, dtype=dtype, seed=6)
+    ref = reference_port.attention_batched(qd.float(), kd.float(), vd.float(),
+                                           softmax_scale=hd ** -0.5, causal=True)
+    out, paged = both_routes(monkeypatch, taken, lambda: mx.flash_attn_func(
+        qd.to(device), kd.to(device), vd.to(device), causal=True))
+    close(out, ref, dtype)
+    assert torch.equal(out, paged)
+
+
+def test_a_sequence_past_4_gib(device, monkeypatch, taken):
+    # Token rows 128 KiB apart: the last ones lie past 2^32 bytes from the first.
+    seq, hd = 34001, 64
+    buf = torch.empty(seq, 65536, dtype=torch.bfloat16, device=device)
+    kv = randn(seq, 2 * hd, dtype=torch.bfloat16, seed=1)
+    buf[:, :2 * hd] = kv.to(device)
+    k, v = (buf[:, i * hd:(i + 1) * hd].unsqueeze(1) for i in (0, 1))
+    q = randn(1, 4, hd, dtype=torch.bfloat16, seed=2)
+    # The last keys outweigh the others, so the output is mostly theirs.
+    q[0, :2] = kv[-1, :hd]
+    ref = reference_port.attention_single(q.float(), kv[:, None, :hd].float(),
+                                          kv[:, None, hd:].float(), softmax_scale=hd ** -0.5)
+    out, paged = both_routes(monkeypatch, taken, lambda: mx.flash_attn_func(
+        q.to(device)[None], k[None], v[None], causal=True))
+    close(out[0], ref, torch.bfloat16)
+    assert torch.equal(out, paged)
+    cu = torch.tensor([0, 100, seq], device=device)
+    got = mx.flash_attn_varlen_func(q.to(device).expand(2, 4, hd).contiguous(), k, v,
+                                    torch.arange(3, device=device), cu, 1, seq)
+    want = reference_port.attention_single(q.float(), kv[100:, None, :hd].float(),
+                                           kv[100:, None, hd:].float(), softmax_scale=hd ** -0.5)
+    close(got[1:], want, torch.bfloat16)
