@@ -216,7 +216,10 @@ py::object decode(const at::Tensor &q, const at::Tensor &k_cache, const at::Tens
 
 // Host copies of a packed call's offsets, written by the call's first (small)
 // launch into pinned memory. get() waits for that launch only, not for the
-// decode behind it, so the caller checks the offsets while the decode runs.
+// decode behind it, so the caller checks the offsets while the decode runs. The
+// event releases the device's writes to the system: torch's pinned memory is
+// coherent by default, but the process may ask for the other kind
+// (HIP_HOST_COHERENT=0), and then nothing else shows the host these values.
 // Against two blocking reads before the launch (each a copy kernel, and the GPU
 // idle until the host had checked and launched), 32 packed sequences of 1k-8k
 // keys, 32q/8kv HD 128, on MI355X: 157.8 -> 117.0 us a call.
@@ -231,7 +234,8 @@ class PackedOffsets {
     if (recorded_ || event_) return false;  // one call each
     n_ = num_seqs + 1;
     values_ = at::empty({2 * n_}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
-    return hipEventCreateWithFlags(&event_, hipEventDisableTiming) == hipSuccess;
+    return hipEventCreateWithFlags(&event_, hipEventDisableTiming | hipEventReleaseToSystem) ==
+           hipSuccess;
   }
   int64_t *memory() {
     void *p = nullptr;
