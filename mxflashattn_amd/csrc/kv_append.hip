@@ -46,9 +46,11 @@ struct AppendParams {
 // slot, then the page id, then the row. All of the arithmetic ran in 64 bits,
 // whose divisions are long software sequences ahead of every load; I = uint32_t
 // (appends of fewer than 2^31 fragments) divides in 32 bits, and positions and
-// slots do too where they fit. Measured on MI355X (us a call): the fp8 append and
-// decode of one layer, 128 sequences of 8 kv heads, HD 128, 77.43 -> 76.97; 8192
-// rows of 8 heads, HD 128, bf16, 11.33 -> 11.20 (6.0 TB/s read and written).
+// slots do too where they fit. Measured on MI355X (us a call, rows of 8 heads, HD
+// 128): into an fp8 cache 2048 rows 5.00 -> 4.49, 8192 12.15 -> 11.49, 32768 37.0
+// -> 35.5; bf16 4096 rows 5.50 -> 5.33, 8192 11.40 -> 11.33 (5.9 TB/s read and
+// written), 32768, bound by memory, 43.3 both. Up to 128 rows the host's 3 us
+// hide it.
 __device__ __forceinline__ void page_of(int64_t pos, int ps, int64_t &page, int64_t &off) {
   if (pos <= 0x7fffffff) {
     const uint32_t q = (uint32_t)pos / (uint32_t)ps;

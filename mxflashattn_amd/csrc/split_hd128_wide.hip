@@ -1,5 +1,5 @@
 // Instantiation unit of the split partial kernel for head dim 128 and more
-// than 16 columns (several query tokens per sequence), two or four groups of
+// than 16 columns (several query tokens per sequence), two or three groups of
 // 16 columns per wave.
 #include "split_kernels.h"
 

@@ -1604,8 +1604,11 @@ __global__ __launch_bounds__(kCombineThreads) void split_combine_kernel(
   }
   block_stamp_after(p, 2, M);
   // One group (a typical batch: at most eight pieces a sequence) has nothing to
-  // merge; without the LDS round trip and its barrier, on MI355X (us a call): 128
-  // short sequences 18.62 -> 18.45, eight verified tokens at B 32 133.4 -> 132.8.
+  // merge; without the LDS round trip and its barriers, on MI355X (us a call): 128
+  // sequences of up to 512 keys, 16q/8kv HD 64, 18.15 -> 17.95; 32 of 800-1024
+  // keys, 32q/8kv HD 128, 24.68 -> 24.45. Calls that merge (1-8 sequences over
+  // many ranges) 6.7-17.1 us, within 0.03 of the kernel without the test (with the
+  // choice made by the host as a template argument too).
   if (groups > 1) {
     float *red = s_red + threadIdx.x * 6;
     red[0] = M;
@@ -1779,10 +1782,6 @@ inline Grid grid_for(int hkv, int num_splits, int waves) {
 template <int HD, bool kF8>
 constexpr int kNbuf = kRowBytes<HD, kF8> <= 64 ? 4 : kRowBytes<HD, kF8> <= 128 ? 3 : 2;
 
-// Register sets of launches of more than 16 columns (several groups per wave).
-template <int HD, bool kF8>
-constexpr int kWideNbuf = kNbuf<HD, kF8>;
-
 // Eight-wave workgroups of 128-byte rows (two waves per SIMD) take two
 // register sets instead of three when the host's bound on tiles per range is
 // small: the shorter pipeline fill and drain pay more than the third set's
@@ -1955,7 +1954,7 @@ inline int launch_columns(int hd, int ps, bool fp8, bool extras) {
 template <int HD, typename T, bool kF8, bool kExtras, int kWaveScan, int kGroups>
 static int launch_wide_g(const DecodeParams &p, const Grid &g, hipStream_t st) {
   const size_t lds = kWaveScan ? 0 : (size_t)(p.batch + 1) * sizeof(int32_t);
-  hipLaunchKernelGGL((split_partial_kernel<HD, 4, T, kF8, false, kWideNbuf<HD, kF8>, 4, kExtras,
+  hipLaunchKernelGGL((split_partial_kernel<HD, 4, T, kF8, false, kNbuf<HD, kF8>, 4, kExtras,
                                            kWaveScan, 0, kGroups>),
                      dim3(g.gx, g.gy), dim3(256), lds, st, p.seqlens, p.batch, p);
   return hipGetLastError() == hipSuccess ? MXFA_OK : MXFA_ELAUNCH;
