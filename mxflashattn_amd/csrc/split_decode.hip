@@ -550,7 +550,8 @@ static int run_tokens(SplitArgs a, int64_t q_stride_t, int q_len, int causal, in
 
 // First rows and lengths of sequences whose keys are consecutive rows, for the
 // decode kernels' block table and lengths. One workgroup: a few hundred to
-// 16,000 entries, latency-bound (about 2 us, where building the same as a
+// 16,000 entries, latency-bound (at least 1.4 us for 16 dense sequences, 3.6 for
+// 32 packed ones with the host's copy, where building the same as a
 // table of one-token pages took four or five elementwise launches and 4 bytes
 // a key). Measured on MI355X against that table and its per-lane page ids (us
 // a call through the API, same outputs bit for bit): 32 packed sequences of

@@ -253,3 +253,32 @@ def test_a_sequence_past_4_gib(device, monkeypatch, taken):
     want = reference_port.attention_single(q.float(), kv[100:, None, :hd].float(),
                                            kv[100:, None, hd:].float(), softmax_scale=hd ** -0.5)
     close(got[1:], want, torch.bfloat16)
+
+
+@pytest.mark.parametrize("ql,seq", [(1, 3001), (16, 3001), (1, 96)])
+def test_dense_keys_from_a_graph(device, taken, ql, seq):
+    # First rows and lengths are memory of the graph; other calls in between,
+    # on the capture's stream and off it, do not change a replay.
+    k, v = (randn(4, seq, 2, 128, dtype=torch.bfloat16, seed=s).to(device) for s in (1, 2))
+    q = randn(4, ql, 8, 128, dtype=torch.bfloat16, seed=3).to(device)
+    stream = torch.cuda.Stream(device)
+    with torch.cuda.stream(stream):
+        want = mx.flash_attn_func(q, k, v, causal=True)
+    torch.cuda.synchronize()
+    taken.clear()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        out = mx.flash_attn_func(q, k, v, causal=True)
+    assert taken == ["contiguous_decode"]
+    cu = torch.tensor([0, 20, seq], device=device)
+    for _ in range(3):
+        out.fill_(7)
+        for s in (stream, torch.cuda.current_stream()):
+            with torch.cuda.stream(s):
+                mx.flash_attn_varlen_func(q[0, 0].expand(2, 8, 128).contiguous(), k[0], v[0],
+                                          torch.arange(3, device=device), cu, 1, seq)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
