@@ -60,12 +60,13 @@ int mxfa_package_decode_tokens_launch(
 //     null) is recorded once they are there, ahead of the decode.
 // rows (2 * batch int32 in device memory): one small launch writes first rows
 // and lengths there (unless rows_written: an earlier launch of the same call
-// did), and the decode reads them. Memory of this call alone: first
-// rows and lengths are held to the rows that exist where they are written, so
-// nothing else (a replay of a graph that holds a workspace) may write them
-// before the decode has read them.
-// page_size: of the pages that hold the same bytes (1 for packed keys); with the
-// splits their heuristic chooses, one token's result is that of those pages.
+// did), and the decode reads them. First rows and lengths are held to the rows
+// that exist where they are written, so nothing else (a replay of a graph that
+// holds this memory) may write them before the decode has read them.
+// page_size: of the pages that hold the same bytes (1 for packed keys). With
+// ranges (num_splits > 0) that their heuristic chooses, one launch gives the bits
+// of those pages; the per-sequence kernel, which pages of less than a tile do not
+// take, gives their error against 64 bits or less.
 // q_len query tokens of at most mxfa_package_launch_columns(head_dim, 16, 0, 0)
 // columns; mxfa_package_contiguous_workspace_size is the workspace of the widest
 // launch of a call of q_len tokens (0 for MXFA_SPLITS_PER_SEQUENCE).

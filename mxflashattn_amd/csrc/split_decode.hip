@@ -68,9 +68,9 @@ int launch_wide_128(const DecodeParams &p, const Grid &g, int dtype, bool fp8, h
 int launch_combine_64(const CombineParams &c, int dtype, hipStream_t st);
 int launch_combine_128(const CombineParams &c, int dtype, hipStream_t st);
 int launch_combine_256(const CombineParams &c, int dtype, hipStream_t st);
-int launch_seq_64(const DecodeParams &p, int dtype, bool fp8, hipStream_t st);
-int launch_seq_128(const DecodeParams &p, int dtype, bool fp8, hipStream_t st);
-int launch_seq_256(const DecodeParams &p, int dtype, bool fp8, hipStream_t st);
+int launch_seq_64(const DecodeParams &p, int dtype, bool fp8, bool each_tile, hipStream_t st);
+int launch_seq_128(const DecodeParams &p, int dtype, bool fp8, bool each_tile, hipStream_t st);
+int launch_seq_256(const DecodeParams &p, int dtype, bool fp8, bool each_tile, hipStream_t st);
 int launch_probe_64(const DecodeParams &p, const Grid &g, int nbuf, uint32_t *sink,
                     hipStream_t st);
 int launch_probe_128(const DecodeParams &p, const Grid &g, int nbuf, uint32_t *sink,
@@ -445,10 +445,11 @@ static int launch_seq(const SplitArgs &a, hipStream_t st) {
   const Grid g = seq_grid(a.hkv, a.batch);
   DecodeParams p = make_params(a, g);
   p.num_ranges = 0;
+  const bool each_tile = a.contiguous && a.same_pages < kTile;
   switch (a.hd) {
-    case 64: return launch_seq_64(p, a.dtype, a.fp8, st);
-    case 128: return launch_seq_128(p, a.dtype, a.fp8, st);
-    default: return launch_seq_256(p, a.dtype, a.fp8, st);
+    case 64: return launch_seq_64(p, a.dtype, a.fp8, each_tile, st);
+    case 128: return launch_seq_128(p, a.dtype, a.fp8, each_tile, st);
+    default: return launch_seq_256(p, a.dtype, a.fp8, each_tile, st);
   }
 }
 

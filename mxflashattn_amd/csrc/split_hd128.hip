@@ -14,8 +14,8 @@ int launch_combine_128(const CombineParams &c, int dtype, hipStream_t st) {
   return launch_combine_hd<128>(c, dtype, st);
 }
 
-int launch_seq_128(const DecodeParams &p, int dtype, bool fp8, hipStream_t st) {
-  return launch_seq_hd<128>(p, dtype, fp8, st);
+int launch_seq_128(const DecodeParams &p, int dtype, bool fp8, bool each_tile, hipStream_t st) {
+  return launch_seq_hd<128>(p, dtype, fp8, each_tile, st);
 }
 
 int launch_probe_128(const DecodeParams &p, const Grid &g, int nbuf, uint32_t *sink,

@@ -14,8 +14,8 @@ int launch_combine_256(const CombineParams &c, int dtype, hipStream_t st) {
   return launch_combine_hd<256>(c, dtype, st);
 }
 
-int launch_seq_256(const DecodeParams &p, int dtype, bool fp8, hipStream_t st) {
-  return launch_seq_hd<256>(p, dtype, fp8, st);
+int launch_seq_256(const DecodeParams &p, int dtype, bool fp8, bool each_tile, hipStream_t st) {
+  return launch_seq_hd<256>(p, dtype, fp8, each_tile, st);
 }
 
 }  // namespace mxfa

@@ -781,9 +781,13 @@ struct Tile {
 // kGroups > 1 (HR 4): up to 16 * kGroups columns. Column 16g + c is column c
 // of group g, with its own QK result, softmax state and PV accumulators; the
 // K and V words of a tile are loaded (and widened or paired) once for all.
+//
+// kEachTile: every tile moves the reference to its own maximum, up or down (by
+// at most kRescaleLog2), so its largest weight is exactly 1 before P is rounded,
+// as in pieces of one tile each.
 template <int HD, int HR, typename T, bool kF8, bool kLanePages, int NBUF, bool kExtras,
           bool kSeq, bool kBalance = false, bool kProbe = false, int kWaveLocal = 0,
-          int kValuG = 0, int kGroups = 1>
+          int kValuG = 0, int kGroups = 1, bool kEachTile = false>
 __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32_t *s_tiles,
                                               int kvh, int rr, int lo, int hi, int stride,
                                               float *lds_o, float *lds_lse, int pg_first = 0,
@@ -1244,7 +1248,9 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
       }
     }
     // The reference moves when a score passes it by more than this.
-    const float move = kTwoExact && after_first ? second_move : kRescaleLog2;
+    const float move = kEachTile                  ? -INFINITY
+                       : kTwoExact && after_first ? second_move
+                                                  : kRescaleLog2;
     after_first = (d.flags & kFirst) != 0;
     uint2 a[kGroups];  // P of each group, packed pairs of the element type
     static_for<kGroups>([&](auto gc) {
@@ -1285,7 +1291,7 @@ __device__ __forceinline__ uint32_t run_range(const DecodeParams &p, const int32
         // Rare, wave-uniform: move the reference of each head to the wave's
         // tile maximum when it passed the reference by more than kRescaleLog2.
         const float mt = rows_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
-        const float to = kTwoExact ? fmaxf(mt, m[g] - kRescaleLog2) : mt;
+        const float to = kTwoExact || kEachTile ? fmaxf(mt, m[g] - kRescaleLog2) : mt;
         const float mn = mt > m[g] + move ? to : m[g];
         const float f = (mn == m[g]) ? 1.f : fast_exp2(m[g] - mn);  // m = -inf: f = 0
         dsum[g] *= f;
@@ -1654,8 +1660,15 @@ __global__ __launch_bounds__(kCombineThreads) void split_combine_kernel(
 // column) in wave order and rounds the output once. Waves past the sequence's
 // tiles leave an LSE of -inf and are skipped; an empty sequence gets zeros.
 // LDS: WAVES * C * (HD + 1) floats, C = GQ * QL.
+//
+// kEachTile (keys in consecutive rows that pages of less than a tile would give
+// to the split kernel, about one tile a piece): run_range's, so that a wave that
+// walks several tiles rounds no more than those pieces do. Error against 64 bits
+// (fp16, HD 64, 8q/2kv, B 4, 500-767 keys; one-token pages 2.45e-4): one
+// reference for a wave's tiles 2.87e-4, one a tile 2.45e-4, in the same time (4
+// dense sequences of 767 keys 15.5 / 15.4 us a call; the split kernel 19.3).
 template <int HD, int HR, typename T, bool kF8, bool kLanePages, int NBUF, int WAVES, int OCC,
-          bool kExtras>
+          bool kExtras, bool kEachTile = false>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC)))
 void seq_decode_kernel(const int32_t *seqlens, const int32_t *bt, int64_t bt_stride, int max_len,
                        int seqlen_add, int ps_log2, DecodeParams p) {
@@ -1701,7 +1714,7 @@ void seq_decode_kernel(const int32_t *seqlens, const int32_t *bt, int64_t bt_str
     v.batch = 1;
     wave_stamp(p, 0, t_entry);
     wave_stamp(p, 1, wave_clock());
-    run_range<HD, HR, T, kF8, kLanePages, NBUF, kExtras, true>(
+    run_range<HD, HR, T, kF8, kLanePages, NBUF, kExtras, true, false, false, 0, 0, 1, kEachTile>(
         v, nullptr, kvh, 0, sub, n, S, s_piece + wave * nc * HD, lse_base + wave * nc, pg_first);
     wave_stamp(p, 3, wave_clock());
     wave_stamp(p, 4, (n - sub + S - 1) / S);
@@ -2033,6 +2046,26 @@ static int launch_seq_t(const DecodeParams &p, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? MXFA_OK : MXFA_ELAUNCH;
 }
 
+// Plain calls on 16-bit keys in consecutive rows (page-uniform tiles).
+template <int HD, int HR, typename T>
+static int launch_seq_each(const DecodeParams &p, hipStream_t st) {
+  hipLaunchKernelGGL((seq_decode_kernel<HD, HR, T, false, false, kNbuf<HD, false>, kSeqWaves,
+                                        kSeqOcc<HD>, false, true>),
+                     dim3(p.hkv, p.batch), dim3(kSeqWaves * 64),
+                     seq_lds_bytes(HD, p.gq * p.ql), st, p.seqlens, p.bt, p.bt_stride, p.max_len,
+                     p.seqlen_add, p.ps_log2, p);
+  return hipGetLastError() == hipSuccess ? MXFA_OK : MXFA_ELAUNCH;
+}
+
+template <int HD, typename T>
+static int launch_seq_each_hr(const DecodeParams &p, hipStream_t st) {
+  switch (head_rows(p.gq * p.ql)) {
+    case 1: return launch_seq_each<HD, 1, T>(p, st);
+    case 2: return launch_seq_each<HD, 2, T>(p, st);
+    default: return launch_seq_each<HD, 4, T>(p, st);
+  }
+}
+
 template <int HD, typename T, bool kF8>
 static int launch_seq_hr(const DecodeParams &p, hipStream_t st) {
   switch (head_rows(p.gq * p.ql)) {
@@ -2043,8 +2076,14 @@ static int launch_seq_hr(const DecodeParams &p, hipStream_t st) {
 }
 
 template <int HD>
-int launch_seq_hd(const DecodeParams &p, int dtype, bool fp8, hipStream_t st) {
+int launch_seq_hd(const DecodeParams &p, int dtype, bool fp8, bool each_tile, hipStream_t st) {
   if (p.heads_per_wg != 1 || p.subs != kSeqWaves) return MXFA_ELAUNCH;  // the kernel's shape
+  if (each_tile) {
+    if (HD > 128 || fp8 || !plain_call(p)) return MXFA_EUNSUPPORTED;  // not instantiated
+    if constexpr (HD <= 128)
+      return dtype == MXFA_DTYPE_BF16 ? launch_seq_each_hr<HD, BF16>(p, st)
+                                      : launch_seq_each_hr<HD, F16>(p, st);
+  }
   if (dtype == MXFA_DTYPE_BF16)
     return fp8 ? launch_seq_hr<HD, BF16, true>(p, st) : launch_seq_hr<HD, BF16, false>(p, st);
   return fp8 ? launch_seq_hr<HD, F16, true>(p, st) : launch_seq_hr<HD, F16, false>(p, st);

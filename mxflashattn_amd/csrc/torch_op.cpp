@@ -74,6 +74,26 @@ at::Tensor workspace(const at::Device &device, void *stream, size_t bytes) {
   return it->second;
 }
 
+// First rows and lengths of a call on keys in consecutive rows: memory that no
+// other call or graph writes before the decode has read it (mxfa_package.h). A
+// graph gets memory of its own pool; eager calls of one stream, which follow each
+// other, share at most 128 KB (16,000 sequences) that no graph holds (an
+// allocation per call cost 1 us of a short call's 15).
+at::Tensor rows_table(const at::Device &device, void *stream, int64_t batch, bool capturing) {
+  const auto options = at::TensorOptions().dtype(at::kInt).device(device);
+  if (capturing) return at::empty({2 * batch}, options);
+  struct Tables {
+    std::mutex mu;
+    std::map<std::pair<int, void *>, at::Tensor> live;
+  };
+  static Tables *tables = new Tables();  // never destroyed, as the workspaces
+  std::lock_guard<std::mutex> lock(tables->mu);
+  at::Tensor &t = tables->live[std::make_pair((int)device.index(), stream)];
+  if (!t.defined() || t.numel() < 2 * batch)
+    t = at::empty({std::max<int64_t>(2 * batch, 1024)}, options);
+  return t;
+}
+
 // MXFA_POISON_OUTPUTS=1 (a debugging aid, read once; the Python binding reads
 // the same variable): outside graph capture the output of a call is filled with
 // NaN and the workspace of each of its launches with 0xff bytes, so a row or a
@@ -296,8 +316,8 @@ py::object contiguous_decode(const at::Tensor &q, const at::Tensor &k, const at:
   const int64_t batch = q.size(0), ql = packed ? 1 : q.size(1);
   const int64_t hq = q.size(-2), hkv = k.size(-2), hd = q.size(-1);
   const int64_t firsts = k.size(0);
-  if (batch < 1 || ql < 1 || hkv < 1 || hq % hkv || hq / hkv > 16 || k.size(-1) != hd ||
-      max_len < 1 || max_len > 1 << 30 || firsts > std::numeric_limits<int>::max())
+  if (batch < 1 || batch > 16000 || ql < 1 || hkv < 1 || hq % hkv || hq / hkv > 16 ||
+      k.size(-1) != hd || max_len < 1 || max_len > 1 << 30 || firsts > std::numeric_limits<int>::max())
     return py::none();
   const auto vector_on_device = [&](const at::Tensor &t) {
     return t.device() == device && t.dim() == 1 && t.is_contiguous();
@@ -350,20 +370,16 @@ py::object contiguous_decode(const at::Tensor &q, const at::Tensor &k, const at:
     out = at::empty(q.sizes(), q.options());
     strides(out, os);
   }
-  // The heuristic as for the pages of the same bytes (decode.py): one-token
-  // pages for packed keys, for a dense cache the largest power of two dividing
-  // its length, up to 256. Asked with pages of 16 it gave short sequences to the
-  // per-sequence kernel, whose waves hold several tiles against one reference
-  // maximum: the largest weight of a tile is then no longer exactly 1 before P
-  // is rounded, and the error against 64 bits grew by up to 19 % (fp16, HD 64,
-  // 8q/2kv, sequences of 500-767 keys: 2.45e-4 -> 2.87e-4; bf16 1.96e-3 ->
-  // 2.30e-3). The split kernel and its second launch cost 1-4 us a call there (32
-  // packed sequences 33.0 -> 34.5 us, 4 dense ones 15.2 -> 19.1 us).
+  // The pages that hold the same bytes (decode.py): one-token pages for packed
+  // keys, for a dense cache of the largest power of two dividing its length, up
+  // to 256. Splits as for those pages, or, pages of less than a tile being read
+  // lane by lane there and as well as any here, as for pages of 16.
   const int64_t len = packed ? 1 : k.size(1);
-  const int ps = (int)std::min<int64_t>(len & -len, 256), width = (int)((max_len + ps - 1) / ps);
+  const int ps = (int)std::min<int64_t>(len & -len, 256), tile = std::max(ps, 16);
+  const int width = (int)((max_len + tile - 1) / tile);
   const int wide = mxfa_package_launch_columns((int)hd, 16, 0, 0);
   int ns = 0;
-  if (mxfa_package_num_splits((int)batch, (int)ql, (int)hq, (int)hkv, (int)hd, ps, width, 0, wide,
+  if (mxfa_package_num_splits((int)batch, (int)ql, (int)hq, (int)hkv, (int)hd, tile, width, 0, wide,
                               num_cus(device.index()), &ns) != MXFA_OK)
     return py::none();
   const int64_t tokens = mxfa_package_tokens_per_launch(
@@ -374,23 +390,20 @@ py::object contiguous_decode(const at::Tensor &q, const at::Tensor &k, const at:
                                              &ws_bytes) != MXFA_OK)
     return py::none();
   void *stream = (void *)c10::hip::getCurrentHIPStream(device.index()).stream();
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)stream, &status) != hipSuccess) return py::none();
+  const bool capturing = status != hipStreamCaptureStatusNone;
+  int64_t *host_offsets = nullptr;
+  // A capture cannot be waited for; the caller reads the offsets another way.
+  if (offsets && (!packed || capturing || !offsets->reserve(num_seqs) ||
+                  !(host_offsets = offsets->memory())))
+    return py::none();
   at::Tensor ws_t;
   if (ws_bytes) ws_t = workspace(device, stream, ws_bytes);
   void *ws = ws_bytes ? ws_t.data_ptr() : nullptr;
   poison(stream, &out, ws_bytes ? &ws_t : nullptr);
-  // First rows and lengths: memory of this call, not the workspace, which
-  // captured graphs write whenever they are replayed.
-  at::Tensor rows_t = at::empty({2 * batch}, q.options().dtype(at::kInt));
+  const at::Tensor rows_t = rows_table(device, stream, batch, capturing);
   const int64_t token_stride = k.stride(packed ? 0 : 1);
-  int64_t *host_offsets = nullptr;
-  if (offsets) {
-    // A capture cannot be waited for; the caller reads the offsets another way.
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (!packed || hipStreamIsCapturing((hipStream_t)stream, &status) != hipSuccess ||
-        status != hipStreamCaptureStatusNone || !offsets->reserve(num_seqs) ||
-        !(host_offsets = offsets->memory()))
-      return py::none();
-  }
   for (int64_t t = 0; t < ql; t += tokens) {
     const int64_t n = std::min(tokens, ql - t);
     if (t > 0) poison(stream, nullptr, ws_bytes ? &ws_t : nullptr);

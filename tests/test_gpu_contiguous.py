@@ -60,29 +60,40 @@ def test_packed_rows(device, monkeypatch, taken, hd, gq, dtype, wide):
     assert torch.equal(out, paged)  # the same tiles, ranges and arithmetic
 
 
-@pytest.mark.parametrize("hd", [64, 128])
-def test_short_packed_sequences_are_split_as_their_pages(device, monkeypatch, taken, hd):
-    # Sequences short enough for the per-sequence kernel, which rounds more
-    # weights against one reference maximum: one-token pages never took it.
-    lens = [1, 16, 200, 255, 31]
-    k, v = (randn(sum(lens), 2, hd, dtype=torch.float16, seed=s) for s in (1, 2))
-    q = randn(5, 8, hd, dtype=torch.float16, seed=3)
-    cu_q, cu_k = torch.arange(6), torch.tensor([0, *torch.tensor(lens).cumsum(0).tolist()])
-    ref = reference_port.attention_varlen(q.float(), k.float(), v.float(), cu_q.tolist(),
-                                          cu_k.tolist(), softmax_scale=hd ** -0.5)
-    out, paged = both_routes(monkeypatch, taken, lambda: mx.flash_attn_varlen_func(
-        q.to(device), k.to(device), v.to(device), cu_q.to(device), cu_k.to(device), 1, 255))
-    close(out, ref, torch.float16)
-    assert torch.equal(out, paged)
-
-
-@pytest.mark.parametrize("seq", [33, 129, 250, 383])  # pages of 1 or 2 tokens
-@pytest.mark.parametrize("hd", [64, 128])
-def test_short_odd_dense_keys_are_split_as_their_pages(device, monkeypatch, taken, seq, hd):
-    k, v = (randn(4, seq, 2, hd, dtype=torch.bfloat16, seed=s).to(device) for s in (1, 2))
-    q = randn(4, 1, 8, hd, dtype=torch.bfloat16, seed=3).to(device)
-    out, paged = both_routes(monkeypatch, taken, lambda: mx.flash_attn_func(q, k, v, causal=True))
-    assert torch.equal(out, paged)
+@pytest.mark.parametrize("hd,dtype", [(64, torch.float16), (64, torch.bfloat16),
+                                      (128, torch.bfloat16)])
+@pytest.mark.parametrize("gq", [1, 4, 8, 16])
+@pytest.mark.parametrize("form", ["packed", "dense"])
+def test_short_sequences_round_no_more_than_their_pages(device, monkeypatch, taken, hd, dtype, gq,
+                                                        form):
+    """Short enough for the per-sequence kernel, which pages of less than a tile
+    never took: a wave of it walks several tiles, where their split has about one
+    a piece. Against 64 bits the error is the rounding of P, sampled over 49,000
+    outputs and more (0.3 % of noise), held to 2 %; with one reference maximum
+    for a wave's tiles it was 8-17 % larger."""
+    lens = [97, 130, 207, 301] if form == "packed" else [301] * 4
+    err = {"rows": 0.0, "pages": 0.0}
+    for seed in range(max(1, 96 // gq)):
+        k, v = (randn(sum(lens), 2, hd, dtype=dtype, seed=2 * seed + i).to(device) for i in (0, 1))
+        q = randn(4, 2 * gq, hd, dtype=dtype, seed=1000 + seed).to(device)
+        if form == "packed":
+            cu_q, cu_k = (torch.tensor([0, *torch.tensor(x).cumsum(0).tolist()], device=device)
+                          for x in ([1] * 4, lens))
+            got = both_routes(monkeypatch, taken, lambda: mx.flash_attn_varlen_func(
+                q, k, v, cu_q, cu_k, 1, max(lens)))
+        else:
+            got = both_routes(monkeypatch, taken, lambda: mx.flash_attn_func(
+                q[:, None], k.unflatten(0, (4, -1)), v.unflatten(0, (4, -1)), causal=True))
+        want, at = [], 0
+        for b, n in enumerate(lens):
+            ki, vi = (t[at:at + n].double().permute(1, 0, 2) for t in (k, v))
+            s = torch.matmul(q[b].double().view(2, gq, hd), ki.transpose(1, 2).contiguous())
+            want.append(torch.matmul(torch.softmax(s * hd ** -0.5, -1), vi.contiguous()))
+            at += n
+        want = torch.stack(want).view(4, 2 * gq, hd)
+        for name, out in zip(err, got):
+            err[name] += (out.view_as(q).double() - want).square().sum().item()
+    assert err["rows"] <= 1.02 ** 2 * err["pages"], err
 
 
 @pytest.mark.parametrize("seq", [1, 15, 47, 96, 1025, 2048])
@@ -208,27 +219,36 @@ def test_packed_offsets_reach_the_host(device):
 # One lane's, four lanes' and the LDS tile scan; past one pass of the rows launch.
 @pytest.mark.parametrize("seqs", [65, 257, 1100])
 @pytest.mark.parametrize("hd,dtype", [(64, torch.float16), (128, torch.bfloat16)])
-def test_many_sequences(device, monkeypatch, taken, seqs, hd, dtype):
+@pytest.mark.parametrize("longest", [59, 801])  # the per-sequence kernel, the split kernel
+def test_many_sequences(device, monkeypatch, taken, seqs, hd, dtype, longest):
     g = torch.Generator().manual_seed(seqs)
     lens = torch.randint(1, 60, (seqs,), generator=g)
     rows = torch.randint(0, 4, (seqs,), generator=g).clamp(max=1)  # a quarter without a row
+    lens[seqs // 2], rows[seqs // 2] = longest, 1
     k, v = (randn(int(lens.sum()), 2, hd, dtype=dtype, seed=s) for s in (1, 2))
     q = randn(int(rows.sum()), 4, hd, dtype=dtype, seed=3)
     cu_q, cu_k = (torch.nn.functional.pad(t.cumsum(0), (1, 0)) for t in (rows, lens))
     ref = reference_port.attention_varlen(q.float(), k.float(), v.float(), cu_q.tolist(),
                                           cu_k.tolist(), softmax_scale=hd ** -0.5)
     out, paged = both_routes(monkeypatch, taken, lambda: mx.flash_attn_varlen_func(
-        q.to(device), k.to(device), v.to(device), cu_q.to(device), cu_k.to(device), 1, 59))
+        q.to(device), k.to(device), v.to(device), cu_q.to(device), cu_k.to(device), 1,
+        int(lens.max())))
     close(out, ref, dtype)
-    assert torch.equal(out, paged)
-    kd, vd = (randn(seqs, 51, 2, hd, dtype=dtype, seed=s) for s in (4, 5))
-    qd = randn(seqs, 1, 4, hd, dtype=dtype, seed=6)
-    ref = reference_port.attention_batched(qd.float(), kd.float(), vd.float(),
+    if longest == 801:
+        assert torch.equal(out, paged)
+    g = torch.Generator(device=device).manual_seed(seqs)
+    kd, vd = (torch.randn(seqs, longest, 1, hd, generator=g, device=device).to(dtype)
+              for _ in range(2))
+    qd = torch.randn(seqs, 1, 4, hd, generator=g, device=device).to(dtype)
+    some = torch.arange(0, seqs, 37, device=device)
+    ref = reference_port.attention_batched(*(t[some].float().cpu() for t in (qd, kd, vd)),
                                            softmax_scale=hd ** -0.5, causal=True)
-    out, paged = both_routes(monkeypatch, taken, lambda: mx.flash_attn_func(
-        qd.to(device), kd.to(device), vd.to(device), causal=True))
-    close(out, ref, dtype)
-    assert torch.equal(out, paged)
+    out, paged = both_routes(monkeypatch, taken, lambda: mx.flash_attn_func(qd, kd, vd,
+                                                                           causal=True))
+    close(out[some], ref, dtype)
+    close(out, paged.cpu(), dtype)
+    if longest == 801:
+        assert torch.equal(out, paged)
 
 
 def test_a_sequence_past_4_gib(device, monkeypatch, taken):
