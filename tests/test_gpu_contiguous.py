@@ -302,3 +302,35 @@ def test_dense_keys_from_a_graph(device, taken, ql, seq):
             graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+def test_calls_on_several_streams_and_threads(device):
+    """First rows and lengths are a stream's own: calls of different sizes in
+    flight on four streams, one thread each, give what they give alone."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    def inputs(i):
+        lens = torch.arange(1 + 3 * i, 41 + 3 * i) * (1 + i) % 300 + 1
+        cu_k = torch.nn.functional.pad(lens.cumsum(0), (1, 0))
+        k, v = (randn(int(lens.sum()), 2, 64, dtype=torch.float16, seed=10 * i + s).to(device)
+                for s in (0, 1))
+        q = randn(40, 4, 64, dtype=torch.float16, seed=10 * i + 2).to(device)
+        return q, k, v, torch.arange(41, device=device), cu_k.to(device), 1, int(lens.max())
+
+    cases = [inputs(i) for i in range(4)]
+    want = [mx.flash_attn_varlen_func(*c) for c in cases]
+    streams = [torch.cuda.Stream(device) for _ in cases]
+    torch.cuda.synchronize()
+
+    def run(i):
+        with torch.cuda.stream(streams[i]):
+            dense = (cases[i][0][None, :1], cases[i][1][None, :77], cases[i][2][None, :77])
+            return [(mx.flash_attn_varlen_func(*cases[i]), mx.flash_attn_func(*dense, causal=True))
+                    for _ in range(25)]
+
+    with ThreadPoolExecutor(4) as pool:
+        got = list(pool.map(run, range(4)))
+    torch.cuda.synchronize()
+    for i, outs in enumerate(got):
+        assert all(torch.equal(packed, want[i]) for packed, _ in outs)
+        assert all(torch.equal(dense, outs[0][1]) for _, dense in outs)
